@@ -20,6 +20,8 @@
 //     The 4 waves merge their (max, sum, O) in LDS; with one split the
 //     workgroup writes the normalised bf16 output directly, otherwise it
 //     writes an fp32 partial (O, max, sum) to the workspace.
+//     Ragged batches share their tokens out evenly over the chip instead
+//     (decode_list_kernel).
 //   pass 2 (decode_combine_kernel): log-sum-exp merge of the partials.
 //
 // Paged KV cache (fgqa_decode_paged): the same kernels read K/V rows through a
@@ -53,7 +55,9 @@ struct DecodeParams {
     int64_t k_sb, k_ss, k_sh;
     int64_t v_sb, v_ss, v_sh;
     int64_t o_sb, o_sh;
-    const int32_t* work;   // ragged work list: [0] = entries, then (b << 16 | split) per entry
+    const int32_t* work;   // ragged work list: [0] = entries, then (b << 16 | split) per entry; or null
+    int64_t* prefix;       // teams: [B + 1] 128-token blocks before each sequence, then their total
+    int teams;             // > 0: the ragged batch's blocks are shared out evenly over this many teams
     int batch, max_seqlen, hq, hkv, group;
     int nsplit, chunk;
     float scale_log2;
@@ -96,34 +100,20 @@ __device__ __forceinline__ int clamp_len(const DecodeParams& p, int b) {
     return min(max(len, 0), p.max_seqlen);
 }
 
-// One (split, kv head, batch) item of pass 1, run by 4 waves (tid: the
-// thread's index among them, smem: their kDecSmemBytes of LDS).  kSeg (paged
+// One item of pass 1: tokens [t_begin, t_end) (not empty) of one sequence and
+// kv head, run by 4 waves (tid: the thread's index among them, smem: their
+// kDecSmemBytes of LDS).  whole: the item is the sequence's only one and
+// writes O and the LSE; otherwise its fp32 partial goes to rows slot0 + head
+// of the workspace.  kSeg (paged
 // caches, 0 or a power of two from one load instruction's rows up to 32): the
 // rows of a 32-token step fall into page segments of kSeg rows
 // (kSeg = min(page, 32)), each read through one buffer resource; 0 is the
 // general form, with a page lookup and a 64-bit address per row.
-// The only workgroup barriers are the two of the wave merge (none when the
-// split is empty), so two items of one split can share a workgroup.
+// The only workgroup barriers are the two of the wave merge, so two items of
+// the same tokens can share a workgroup.
 template <int kKv, int kSeg = 0>
-__device__ __forceinline__ void dec_item(const DecodeParams& p, unsigned char* smem, int split, int kvh, int b,
-                                         int tid) {
-    const int len = clamp_len(p, b);
-    const int t_begin = split * p.chunk;
-    if (t_begin >= len) {
-        // Empty split: the combine never reads it.  Without a combine pass an
-        // empty sequence still needs its O = 0, lse = -inf written here.
-        if (p.nsplit == 1 && (tid >> 4) < p.group) {
-            const int qh = kvh * p.group + (tid >> 4);
-            bf16x8_t z;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) z[j] = (__bf16)0.f;
-            *reinterpret_cast<bf16x8_t*>(p.o + b * p.o_sb + qh * p.o_sh + (tid & 15) * 8) = z;
-            if (p.lse != nullptr && (tid & 15) == 0) p.lse[(int64_t)b * p.hq + qh] = -INFINITY;
-        }
-        return;
-    }
-    const int t_end = min(t_begin + p.chunk, len);
-
+__device__ __forceinline__ void dec_item(const DecodeParams& p, unsigned char* smem, int t_begin, int t_end, int kvh,
+                                         int b, int tid, bool whole, int64_t slot0) {
     const int lane = tid & (kWave - 1);
     constexpr bool kUni = kSeg > 0;
     const int wave = kUni ? __builtin_amdgcn_readfirstlane(tid / kWave) : tid / kWave;
@@ -413,7 +403,7 @@ __device__ __forceinline__ void dec_item(const DecodeParams& p, unsigned char* s
         for (int j = 0; j < 8; ++j) acc[j] += c * src[j];
     }
     const int qh = kvh * p.group + h;
-    if (p.nsplit == 1) {
+    if (whole) {
         const float inv = p.v_scale / L;
         bf16x8_t out;
 #pragma unroll
@@ -421,7 +411,7 @@ __device__ __forceinline__ void dec_item(const DecodeParams& p, unsigned char* s
         *reinterpret_cast<bf16x8_t*>(p.o + b * p.o_sb + qh * p.o_sh + d0) = out;
         if (p.lse != nullptr && (tid & 15) == 0) p.lse[(int64_t)b * p.hq + qh] = M * kLn2 + logf(L);
     } else {
-        const int64_t slot = (((int64_t)b * p.hkv + kvh) * p.nsplit + split) * p.group + h;
+        const int64_t slot = slot0 + h;
         float* po = p.part_o + slot * kHeadDim + d0;
         const float vs = p.v_scale;
         *reinterpret_cast<f32x4_t*>(po) = f32x4_t{acc[0] * vs, acc[1] * vs, acc[2] * vs, acc[3] * vs};
@@ -443,33 +433,53 @@ template <bool kPair>
 __global__ __launch_bounds__(kPair ? 2 * kDecThreads : kDecThreads) void decode_split_kernel(DecodeParams p) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[(kPair ? 2 : 1) * kDecSmemBytes];
     const int half = kPair ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kDecThreads)) : 0;
-    dec_item<kKvContig>(p, smem + half * kDecSmemBytes, blockIdx.x, kPair ? 2 * (int)blockIdx.y + half : blockIdx.y,
-                        blockIdx.z, (int)threadIdx.x - half * kDecThreads);
+    const int tid = (int)threadIdx.x - half * kDecThreads;
+    const int kvh = kPair ? 2 * (int)blockIdx.y + half : blockIdx.y;
+    const int split = blockIdx.x, b = blockIdx.z;
+    const int len = clamp_len(p, b);
+    const int t_begin = split * p.chunk;
+    if (t_begin >= len) {
+        // Empty split: the combine never reads it.  Without a combine pass an
+        // empty sequence still needs its O = 0, lse = -inf written here.
+        if (p.nsplit == 1 && (tid >> 4) < p.group) {
+            const int qh = kvh * p.group + (tid >> 4);
+            bf16x8_t z;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) z[j] = (__bf16)0.f;
+            *reinterpret_cast<bf16x8_t*>(p.o + b * p.o_sb + qh * p.o_sh + (tid & 15) * 8) = z;
+            if (p.lse != nullptr && (tid & 15) == 0) p.lse[(int64_t)b * p.hq + qh] = -INFINITY;
+        }
+        return;
+    }
+    dec_item<kKvContig>(p, smem + half * kDecSmemBytes, t_begin, min(t_begin + p.chunk, len), kvh, b, tid,
+                        p.nsplit == 1, (((int64_t)b * p.hkv + kvh) * p.nsplit + split) * p.group);
 }
 
-// Ragged batches: build the work list of non-empty splits, full-length splits
-// first and the partial last split of each sequence after them, longest first
-// (batch order beyond kPlanSortMax sequences), so that equal work fills the
-// GPU and the short items form the tail.  One workgroup; entry =
-// (b << 16) | split, so batch < 2^15 and splits < 2^16 (checked on the host).
+// Ragged batches with a split length given by the caller: build the work list
+// of non-empty splits, full-length splits first and the partial last split of
+// each sequence after them, longest first (batch order beyond kPlanSortMax
+// sequences), so that equal work fills the GPU and the short items form the
+// tail.  One workgroup; entry = (b << 16) | split, so batch < 2^15 and splits
+// < 2^16 (checked on the host).
 constexpr int kPlanThreads = 256;
 constexpr int kPlanSortMax = 1024;   // remainders kept in LDS and length-sorted up to this batch size
 
-// Exclusive prefix sum of one int per thread over the workgroup (256 threads).
-__device__ __forceinline__ int block_exclusive_scan(int v, int* s_wave, int* total) {
+// Exclusive prefix sum of one value per thread over a workgroup of kThreads.
+template <int kThreads, typename T>
+__device__ __forceinline__ T block_exclusive_scan(T v, T* s_wave, T* total) {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    int incl = v;
+    T incl = v;
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
-        const int t = __shfl_up(incl, d, kWave);
+        const T t = __shfl_up(incl, d, kWave);
         if (lane >= d) incl += t;
     }
     if (lane == kWave - 1) s_wave[wave] = incl;
     __syncthreads();
-    int base = 0, all = 0;
+    T base = 0, all = 0;
 #pragma unroll
-    for (int w = 0; w < kPlanThreads / kWave; ++w) {
+    for (int w = 0; w < kThreads / kWave; ++w) {
         base += (w < wave) ? s_wave[w] : 0;
         all += s_wave[w];
     }
@@ -492,8 +502,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(DecodeParams 
         if (sort) s_rem[b] = len % p.chunk;
     }
     int n_full, n_part;
-    int pos_f = block_exclusive_scan(nf, s_wave, &n_full);
-    int pos_p = block_exclusive_scan(np, s_wave, &n_part);   // also publishes s_rem (barriers inside)
+    int pos_f = block_exclusive_scan<kPlanThreads>(nf, s_wave, &n_full);
+    int pos_p = block_exclusive_scan<kPlanThreads>(np, s_wave, &n_part);   // also publishes s_rem (barriers inside)
     if (tid == 0) work[0] = n_full + n_part;
     for (int b = tid; b < p.batch; b += kPlanThreads) {
         const int len = clamp_len(p, b);
@@ -530,99 +540,240 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(DecodeParams 
     }
 }
 
-// Pass 1 over the ragged work list: a fixed grid walks the entries, each
-// entry once per kv head (kv head fastest, so heads of one split run together).
+// Pass 1 over a ragged batch.  A sequence is a run of 128-token blocks (one
+// pass of 4 waves); team t of n takes blocks [total * t / n, total * (t + 1) /
+// n) of the concatenated sequences, one workgroup per kv head or head pair, so
+// every CU streams the same number of tokens whatever the lengths, and the
+// workgroups of a team read the same rows side by side.  A team's range is cut
+// at the sequences' ends into items; a sequence inside one range is written
+// directly, and only the (at most two per team) items of a sequence that
+// crosses a range's end leave partials: slot 2t for one that starts inside the
+// sequence, 2t + 1 for the sequence's first.  Each workgroup finds its range
+// by itself from the lengths (a scan of one value per thread), which needs no
+// planning launch before it.  Against 4096-token splits handed out by a
+// planning kernel's work list: 8 sequences of up to 6000 tokens, Hq = 32,
+// Hkv = 8, bf16 pages: 88.5 -> 30.3 us; 64 of up to 32768, Hq = 64, fp8 pages:
+// 395.8 -> 360.9 us.
+//
+// A split length given by the caller keeps the work list (p.work): a fixed
+// grid walks its entries, each once per kv head or pair (the head fastest, so
+// heads of one split run together).
+//
 // kPair (an even number of kv heads): 8-wave workgroups, waves 0-3 on kv head
-// 2j and waves 4-7 on kv head 2j + 1 of the same split.  Each half reads its
+// 2j and waves 4-7 on kv head 2j + 1 of the same tokens.  Each half reads its
 // own head's rows, but the two halves' loads of one token arrive together, so
 // the 2 x 128-byte (fp8) or 2 x 256-byte (bf16) pieces of a cache row that lie
 // side by side in memory are read at the same time: a streaming read of
 // config 3's fp8 page pattern ran at 5.84 TB/s with one head per workgroup and
-// 6.45 TB/s with head pairs.  Both halves of a workgroup hold the same split
+// 6.45 TB/s with head pairs.  Both halves of a workgroup hold the same tokens
 // of the same sequence, so they pass the same workgroup barriers.
+__device__ __forceinline__ int64_t team_start(int64_t total, int teams, int t) { return total * t / teams; }
+
+// Teams that get blocks: every one of them at least one.
+__device__ __forceinline__ int team_count(const DecodeParams& p, int64_t total) {
+    return total < p.teams ? (int)total : p.teams;
+}
+
+__device__ __forceinline__ int seq_blocks(int len) {
+    return (len + plan::kDecodeStepRound - 1) / plan::kDecodeStepRound;
+}
+
 template <int kKv, int kSeg = 0, bool kPair = false>
 __global__ __launch_bounds__(kPair ? 2 * kDecThreads : kDecThreads) void decode_list_kernel(DecodeParams p) {
+    constexpr int kThreads = kPair ? 2 * kDecThreads : kDecThreads;
     __shared__ __attribute__((aligned(16))) unsigned char smem[(kPair ? 2 : 1) * kDecSmemBytes];
     // wave-uniform (readfirstlane), so the buffer resources built from the
     // head stay scalar
     const int half = kPair ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kDecThreads)) : 0;
     const int per_entry = kPair ? p.hkv / 2 : p.hkv;
-    const int total = p.work[0] * per_entry;
-    for (int item = blockIdx.x; item < total; item += gridDim.x) {
-        const int e = p.work[1 + item / per_entry];
-        const int kvh = kPair ? 2 * (item % per_entry) + half : item % per_entry;
+    const int tid = (int)threadIdx.x - half * kDecThreads;
+    // work list: items blockIdx.x, + gridDim.x, ...
+    int item = blockIdx.x;
+    const int n_items = p.work != nullptr ? p.work[0] * per_entry : 0;
+    // teams: blocks [g0, g1) of the batch, the first of them block `blk` of sequence b
+    const int team = blockIdx.x / per_entry;
+    int64_t g0 = 0, g1 = 0;
+    int b = 0, blk = 0;
+    if (p.work == nullptr) {
+        int64_t* s_wave = reinterpret_cast<int64_t*>(smem);
+        int* s_pos = reinterpret_cast<int*>(s_wave + kThreads / kWave);
+        const int per = (p.batch + kThreads - 1) / kThreads;
+        const int b_lo = min((int)threadIdx.x * per, p.batch), b_hi = min(b_lo + per, p.batch);
+        int64_t sum = 0, total;
+        for (int i = b_lo; i < b_hi; ++i) sum += seq_blocks(clamp_len(p, i));
+        int64_t at = block_exclusive_scan<kThreads>(sum, s_wave, &total);
+        // (uniform: the compiler does not see it through the LDS sum)
+        total = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(total >> 32)) << 32) |
+                          (uint32_t)__builtin_amdgcn_readfirstlane((int)total));
+        const int teams = team_count(p, total);
+        if (team < teams) {
+            g0 = team_start(total, teams, team);
+            g1 = team_start(total, teams, team + 1);
+        }
+        const bool here = g0 >= at && g0 < at + sum;   // exactly one thread's, unless g0 is the end
+        if (here || blockIdx.x == 0) {
+            for (int i = b_lo; i < b_hi; ++i) {
+                const int n = seq_blocks(clamp_len(p, i));
+                if (blockIdx.x == 0) p.prefix[i] = at;
+                if (g0 >= at && g0 < at + n) {
+                    s_pos[0] = i;
+                    s_pos[1] = (int)(g0 - at);
+                }
+                at += n;
+            }
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) p.prefix[p.batch] = total;
+        if (g0 >= g1) return;
+        __syncthreads();
+        b = __builtin_amdgcn_readfirstlane(s_pos[0]);
+        blk = __builtin_amdgcn_readfirstlane(s_pos[1]);
+    }
+    while (true) {
+        int kvh, t_begin, t_end;
+        bool whole;
+        int64_t slot;
+        if (p.work != nullptr) {
+            if (item >= n_items) break;
+            const int e = p.work[1 + item / per_entry];
+            kvh = item % per_entry;
+            const int split = e & 0xffff;
+            b = e >> 16;
+            t_begin = split * p.chunk;
+            t_end = min(t_begin + p.chunk, clamp_len(p, b));
+            whole = p.nsplit == 1;
+            kvh = kPair ? 2 * kvh + half : kvh;
+            slot = ((int64_t)b * p.hkv + kvh) * p.nsplit + split;
+            item += gridDim.x;
+        } else {
+            if (g0 >= g1) break;
+            const int len = clamp_len(p, b);
+            const int nb = seq_blocks(len);
+            if (nb == 0) {   // empty sequences: the combine writes their O
+                ++b;
+                continue;
+            }
+            const int n = (int)min((int64_t)(nb - blk), g1 - g0);
+            t_begin = blk * plan::kDecodeStepRound;
+            t_end = min((blk + n) * plan::kDecodeStepRound, len);
+            whole = n == nb;
+            kvh = blockIdx.x % per_entry;
+            kvh = kPair ? 2 * kvh + half : kvh;
+            slot = (int64_t)(2 * team + (blk == 0 ? 1 : 0)) * p.hkv + kvh;
+        }
         __syncthreads();   // the previous item's merge buffers alias the staging area
-        dec_item<kKv, kSeg>(p, smem + half * kDecSmemBytes, e & 0xffff, kvh, e >> 16,
-                            (int)threadIdx.x - half * kDecThreads);
+        dec_item<kKv, kSeg>(p, smem + half * kDecSmemBytes, t_begin, t_end, kvh, b, tid, whole, slot * p.group);
+        if (p.work == nullptr) {
+            g0 += (t_end - t_begin + plan::kDecodeStepRound - 1) / plan::kDecodeStepRound;
+            ++b;
+            blk = 0;
+        }
     }
 }
 
-// Launches pass 1 over the work list: the head-pair form (one 8-wave
+// Launches pass 1 over a ragged batch: the head-pair form (one 8-wave
 // workgroup per CU) when the kv heads pair up, else two 4-wave workgroups per
 // CU.  Persistent: the grid never exceeds what the CUs hold at once.
 template <int kKv, int kSeg>
 static void launch_list(const DecodeParams& p, int nsplit, int cus, hipStream_t s) {
     const bool pair = (p.hkv % 2) == 0;
-    const int64_t items = (int64_t)p.batch * nsplit * (pair ? p.hkv / 2 : p.hkv);   // most the list can hold
+    const int per_entry = pair ? p.hkv / 2 : p.hkv;
+    const int64_t items = (int64_t)p.batch * nsplit * per_entry;   // most the list can hold
     const int64_t slots = (int64_t)(pair ? 1 : 2) * cus;
-    const int grid = (int)(items < slots ? items : slots);
+    const int grid = p.teams > 0 ? p.teams * per_entry : (int)(items < slots ? items : slots);
     if (pair)
         hipLaunchKernelGGL((decode_list_kernel<kKv, kSeg, true>), dim3(grid), dim3(2 * kDecThreads), 0, s, p);
     else
         hipLaunchKernelGGL((decode_list_kernel<kKv, kSeg, false>), dim3(grid), dim3(kDecThreads), 0, s, p);
 }
 
-// Log-sum-exp merge of the per-split partials of one (kv head, batch).
+// Log-sum-exp merge of the partials of each (sequence, query head): 16 lanes
+// of 8 dims each x kWays ways, way w taking partials w, w + kWays, ... (in
+// batches of kCombineBatch whose loads are all issued before any is used:
+// slots past the last re-read it and are masked), then one merge of the ways
+// through LDS.  A workgroup holds 16 / kWays heads.  The launch is bound by
+// memory round trips, one per batch, so the host picks as many ways as one
+// batch each needs (combine_ways).  With one way per head at 128 partials (one
+// 32768-token sequence, Hq = 64, Hkv = 8): 27.4 us; 16 ways: 4.3 us.
+template <bool kTeam, int kWays>
 __global__ __launch_bounds__(kDecThreads) void decode_combine_kernel(DecodeParams p) {
-    const int kvh = blockIdx.x;
+    constexpr int kHeads = 16 / kWays;
+    __shared__ float s_part[kWays > 1 ? kWays * kHeads * 16 * 10 : 1];   // acc[8], max, sum per lane
     const int b = blockIdx.y;
-    const int tid = threadIdx.x;
-    const int h = tid >> 4;
-    const int d0 = (tid & 15) * 8;
-    if (h >= p.group) return;
+    const int d16 = threadIdx.x & 15;
+    const int d0 = d16 * 8;
+    const int way = (threadIdx.x >> 4) / kHeads;
+    const int hl = (threadIdx.x >> 4) % kHeads;
+    const int qh_raw = blockIdx.x * kHeads + hl;
+    const int qh = min(qh_raw, p.hq - 1);   // lanes past the last head repeat it and store nothing
+    const int kvh = qh / p.group;
+    const int h = qh - kvh * p.group;
     const int len = clamp_len(p, b);
-    const int nvalid = (len + p.chunk - 1) / p.chunk;
-    const int qh = kvh * p.group + h;
+    // partial i: row base + i * step of the workspace (teams: the first one apart)
+    int n;
+    int64_t first, base, step;
+    if constexpr (kTeam) {
+        n = 0;
+        first = base = step = 0;
+        if (len > 0) {
+            const int64_t total = p.prefix[p.batch], g0 = p.prefix[b], g1 = g0 + seq_blocks(len);
+            const int teams = team_count(p, total);
+            auto team_of = [&](int64_t g) {   // the last team whose start is at most g
+                int t = (int)(g * teams / total);
+                while (t + 1 < teams && team_start(total, teams, t + 1) <= g) ++t;
+                return t;
+            };
+            const int t0 = team_of(g0), t1 = team_of(g1 - 1);
+            if (t0 == t1) return;   // the whole workgroup: pass 1 wrote the sequence's output
+            n = t1 - t0 + 1;
+            first = ((int64_t)(2 * t0 + 1) * p.hkv + kvh) * p.group + h;
+            step = (int64_t)2 * p.hkv * p.group;
+            base = (int64_t)t0 * step + kvh * p.group + h;
+        }
+    } else {
+        n = (len + p.chunk - 1) / p.chunk;
+        step = p.group;
+        first = base = ((int64_t)b * p.hkv + kvh) * p.nsplit * p.group + h;
+    }
     __bf16* orow = p.o + b * p.o_sb + qh * p.o_sh + d0;
-    if (nvalid == 0) {
+    const bool store = way == 0 && qh_raw < p.hq;
+    if (n == 0) {   // (the whole workgroup)
         bf16x8_t z;
 #pragma unroll
         for (int j = 0; j < 8; ++j) z[j] = (__bf16)0.f;
-        *reinterpret_cast<bf16x8_t*>(orow) = z;
-        if (p.lse != nullptr && (tid & 15) == 0) p.lse[(int64_t)b * p.hq + qh] = -INFINITY;
+        if (store) *reinterpret_cast<bf16x8_t*>(orow) = z;
+        if (store && p.lse != nullptr && d16 == 0) p.lse[(int64_t)b * p.hq + qh] = -INFINITY;
         return;
     }
-    const int64_t base = ((int64_t)b * p.hkv + kvh) * p.nsplit;
-    // Splits in batches of kCombineBatch whose loads are all issued before any
-    // is used (slots past the last valid split re-read it and are masked), so
-    // a batch costs one memory round trip; the sums run in split order.
+    auto row_of = [&](int i) {
+        const int c = min(i, n - 1);
+        return c == 0 ? first : base + c * step;
+    };
     constexpr int kCombineBatch = 8;
-    float M = -INFINITY;
-    for (int s0 = 0; s0 < nvalid; s0 += kCombineBatch) {
-        float mv[kCombineBatch];
-#pragma unroll
-        for (int i = 0; i < kCombineBatch; ++i)
-            mv[i] = p.part_ml[((base + min(s0 + i, nvalid - 1)) * p.group + h) * 2];
-#pragma unroll
-        for (int i = 0; i < kCombineBatch; ++i) M = fmaxf(M, mv[i]);
-    }
-    float L = 0.f;
+    float M = -INFINITY, L = 0.f;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < nvalid; s0 += kCombineBatch) {
+    for (int s0 = way; s0 < n; s0 += kCombineBatch * kWays) {
         float ms[kCombineBatch], ls[kCombineBatch];
         f32x4_t a[kCombineBatch], bb[kCombineBatch];
 #pragma unroll
         for (int i = 0; i < kCombineBatch; ++i) {
-            const int64_t slot = (base + min(s0 + i, nvalid - 1)) * p.group + h;
+            const int64_t slot = row_of(s0 + i * kWays);
             ms[i] = p.part_ml[slot * 2];
             ls[i] = p.part_ml[slot * 2 + 1];
             a[i] = *reinterpret_cast<const f32x4_t*>(p.part_o + slot * kHeadDim + d0);
             bb[i] = *reinterpret_cast<const f32x4_t*>(p.part_o + slot * kHeadDim + d0 + 4);
         }
+        float m_new = M;
+#pragma unroll
+        for (int i = 0; i < kCombineBatch; ++i) m_new = fmaxf(m_new, ms[i]);
+        const float c0 = (M == -INFINITY) ? 0.f : fast_exp2(M - m_new);
+        L *= c0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] *= c0;
+        M = m_new;
         // selects, not a branch, so the loads above stay ahead of every use
 #pragma unroll
         for (int i = 0; i < kCombineBatch; ++i) {
-            const bool valid = s0 + i < nvalid;
+            const bool valid = s0 + i * kWays < n;
             const float c = (ms[i] == -INFINITY) ? 0.f : fast_exp2(ms[i] - M);
             L = valid ? L + c * ls[i] : L;
 #pragma unroll
@@ -632,12 +783,68 @@ __global__ __launch_bounds__(kDecThreads) void decode_combine_kernel(DecodeParam
             }
         }
     }
+    if constexpr (kWays > 1) {
+        // [way][head][value][lane]
+        float* mine = s_part + (way * kHeads + hl) * 160 + d16;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mine[j * 16] = acc[j];
+        mine[128] = M;
+        mine[144] = L;
+        __syncthreads();
+        if (way != 0) return;
+        const int nw = min(kWays, n);   // ways that held a partial
+        const float m0 = M;
+        for (int w = 1; w < nw; ++w) M = fmaxf(M, s_part[(w * kHeads + hl) * 160 + 128 + d16]);
+        const float c0 = (m0 == -INFINITY) ? 0.f : fast_exp2(m0 - M);
+        L *= c0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] *= c0;
+        for (int w = 1; w < nw; ++w) {
+            const float* o = s_part + (w * kHeads + hl) * 160 + d16;
+            const float c = (o[128] == -INFINITY) ? 0.f : fast_exp2(o[128] - M);
+            L += c * o[144];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] += c * o[j * 16];
+        }
+    }
+    if (!store) return;
     const float inv = 1.f / L;
     bf16x8_t out;
 #pragma unroll
     for (int j = 0; j < 8; ++j) out[j] = (__bf16)(acc[j] * inv);
     *reinterpret_cast<bf16x8_t*>(orow) = out;
-    if (p.lse != nullptr && (tid & 15) == 0) p.lse[(int64_t)b * p.hq + qh] = M * kLn2 + logf(L);
+    if (p.lse != nullptr && d16 == 0) p.lse[(int64_t)b * p.hq + qh] = M * kLn2 + logf(L);
+}
+
+// Ways of the combine for `n` partials per (sequence, head): one batch of 8
+// each, as far as 16 ways go (a ragged batch's n is the average sequence's,
+// and a long one among short ones has more: 4 ways at least).
+template <bool kTeam>
+static void launch_combine(const DecodeParams& p, int64_t n, hipStream_t s) {
+    if (n > 32)
+        hipLaunchKernelGGL((decode_combine_kernel<kTeam, 16>), dim3(p.hq, p.batch), dim3(kDecThreads), 0, s, p);
+    else if (kTeam || n > 8)
+        hipLaunchKernelGGL((decode_combine_kernel<kTeam, 4>), dim3((p.hq + 3) / 4, p.batch), dim3(kDecThreads), 0, s,
+                           p);
+    else if constexpr (!kTeam)
+        hipLaunchKernelGGL((decode_combine_kernel<false, 1>), dim3((p.hq + 15) / 16, p.batch), dim3(kDecThreads), 0, s,
+                           p);
+}
+
+// The passes over a ragged batch (teams, or the work list of a given split length).
+template <typename Launch>
+static void run_ragged(const DecodeParams& p, int32_t* work, Launch&& pass1, hipStream_t s) {
+    if (p.teams > 0) {
+        pass1();
+        // a sequence's share of the teams if it were the batch's average
+        const int64_t blocks = ceil_div(p.max_seqlen, plan::kDecodeStepRound);
+        const int64_t share = ceil_div(p.teams, p.batch) + 1;
+        launch_combine<true>(p, share < blocks ? share : blocks, s);
+        return;
+    }
+    hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, p, work);
+    pass1();
+    if (p.nsplit > 1) launch_combine<false>(p, p.nsplit, s);
 }
 
 // One pass of the 4 decode waves covers the planner's split rounding.
@@ -646,6 +853,26 @@ static_assert(kDecWaves * kDecStep == plan::kDecodeStepRound, "decode split roun
 namespace {
 using plan::DecodePlan;
 using plan::DecodeShape;
+
+// Points p's partials, and the teams' prefix or the work list (returned, also
+// in p.work), into the workspace.
+int32_t* carve_workspace(const DecodePlan& plan, void* ws, DecodeParams* p) {
+    char* w = static_cast<char*>(ws);
+    if (plan.teams > 0) {
+        p->teams = plan.teams;
+        p->prefix = reinterpret_cast<int64_t*>(w + plan.team_prefix_off);
+        p->part_o = reinterpret_cast<float*>(w);
+        p->part_ml = reinterpret_cast<float*>(w + plan.team_ml_off);
+        return nullptr;
+    }
+    if (plan.nsplit > 1) {
+        p->part_o = reinterpret_cast<float*>(w);
+        p->part_ml = reinterpret_cast<float*>(w + plan.part_o_bytes);
+    }
+    int32_t* work = plan.list ? reinterpret_cast<int32_t*>(w + plan.part_o_bytes + plan.part_ml_bytes) : nullptr;
+    p->work = work;
+    return work;
+}
 
 // The split plan of a validated call on the current device.
 int plan_on_device(const DecodeShape& shape, DecodePlan* pl) {
@@ -729,6 +956,9 @@ int decode_run(const fgqa_decode_args* a, void* stream, bool noalloc) {
     p.seqlens = a->seqlens;
     p.part_o = nullptr;
     p.part_ml = nullptr;
+    p.work = nullptr;
+    p.prefix = nullptr;
+    p.teams = 0;
     p.q_sb = a->q_stride[0];
     p.q_sh = a->q_stride[1];
     p.k_sb = a->k_stride[0];
@@ -767,27 +997,17 @@ int decode_run(const fgqa_decode_args* a, void* stream, bool noalloc) {
         } else if (!aligned16(ws)) {
             return FGQA_ERR_UNSUPPORTED;
         }
-        char* w = static_cast<char*>(ws);
-        if (plan.nsplit > 1) {
-            p.part_o = reinterpret_cast<float*>(w);
-            p.part_ml = reinterpret_cast<float*>(w + plan.part_o_bytes);
-        }
-        if (plan.list) work = reinterpret_cast<int32_t*>(w + plan.part_o_bytes + plan.part_ml_bytes);
+        work = carve_workspace(plan, ws, &p);
     }
-    p.work = work;
 
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (a->max_seqlen == 0) {
         // Every sequence is empty: the combine writes O = 0, lse = -inf.
-        p.nsplit = 1;
-        hipLaunchKernelGGL(decode_combine_kernel, dim3(p.hkv, p.batch), dim3(kDecThreads), 0, s, p);
+        launch_combine<false>(p, 1, s);
     } else if (plan.list) {
         const int cus = device_cu_count();
         if (cus <= 0) return FGQA_ERR_HIP;
-        hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, p, work);
-        launch_list<kKvContig, 0>(p, plan.nsplit, cus, s);
-        if (plan.nsplit > 1)
-            hipLaunchKernelGGL(decode_combine_kernel, dim3(p.hkv, p.batch), dim3(kDecThreads), 0, s, p);
+        run_ragged(p, work, [&] { launch_list<kKvContig, 0>(p, plan.nsplit, cus, s); }, s);
     } else {
         // Head pairs once the grid holds at least one item per CU; smaller
         // grids are latency-bound and keep one item per workgroup (BASELINE
@@ -800,8 +1020,7 @@ int decode_run(const fgqa_decode_args* a, void* stream, bool noalloc) {
                                s, p);
         else
             hipLaunchKernelGGL(decode_split_kernel<false>, dim3(p.nsplit, p.hkv, p.batch), dim3(kDecThreads), 0, s, p);
-        if (plan.nsplit > 1)
-            hipLaunchKernelGGL(decode_combine_kernel, dim3(p.hkv, p.batch), dim3(kDecThreads), 0, s, p);
+        if (plan.nsplit > 1) launch_combine<false>(p, plan.nsplit, s);
     }
     if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
     return FGQA_OK;
@@ -848,6 +1067,9 @@ extern "C" int fgqa_decode_paged(const fgqa_decode_paged_args* a, void* stream) 
     p.seqlens = a->seqlens;
     p.part_o = nullptr;
     p.part_ml = nullptr;
+    p.work = nullptr;
+    p.prefix = nullptr;
+    p.teams = 0;
     p.q_sb = a->q_stride[0];
     p.q_sh = a->q_stride[1];
     p.k_sb = a->k_stride[0];
@@ -887,23 +1109,15 @@ extern "C" int fgqa_decode_paged(const fgqa_decode_paged_args* a, void* stream) 
         } else if (!aligned16(ws)) {
             return FGQA_ERR_UNSUPPORTED;
         }
-        char* w = static_cast<char*>(ws);
-        if (plan.nsplit > 1) {
-            p.part_o = reinterpret_cast<float*>(w);
-            p.part_ml = reinterpret_cast<float*>(w + plan.part_o_bytes);
-        }
-        if (plan.list) work = reinterpret_cast<int32_t*>(w + plan.part_o_bytes + plan.part_ml_bytes);
+        work = carve_workspace(plan, ws, &p);
     }
-    p.work = work;
 
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (a->max_seqlen == 0) {
-        p.nsplit = 1;
-        hipLaunchKernelGGL(decode_combine_kernel, dim3(p.hkv, p.batch), dim3(kDecThreads), 0, s, p);
+        launch_combine<false>(p, 1, s);
     } else {
         const int cus = device_cu_count();
         if (cus <= 0) return FGQA_ERR_HIP;
-        hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, p, work);
         // Pages of at least one load instruction's rows (4 bf16, 8 fp8) whose
         // bytes stay below 2^31: page segments of min(page, 32) rows, each
         // read through one buffer resource (at BASELINE config 3's lengths
@@ -913,24 +1127,25 @@ extern "C" int fgqa_decode_paged(const fgqa_decode_paged_args* a, void* stream) 
         const bool small_pages = (int64_t)a->page_size * a->k_stride[1] * 2 < ((int64_t)1 << 31) &&
                                  (int64_t)a->page_size * a->v_stride[1] * 2 < ((int64_t)1 << 31);
         const int seg = !small_pages ? 0 : a->page_size >= 32 ? 32 : a->page_size >= 4 ? a->page_size : 0;
-        if (fp8) {
-            switch (seg >= 8 ? seg : 0) {
-                case 32: launch_list<kKvPagedFp8, 32>(p, plan.nsplit, cus, s); break;
-                case 16: launch_list<kKvPagedFp8, 16>(p, plan.nsplit, cus, s); break;
-                case 8: launch_list<kKvPagedFp8, 8>(p, plan.nsplit, cus, s); break;
-                default: launch_list<kKvPagedFp8, 0>(p, plan.nsplit, cus, s); break;
+        auto pass1 = [&] {
+            if (fp8) {
+                switch (seg >= 8 ? seg : 0) {
+                    case 32: launch_list<kKvPagedFp8, 32>(p, plan.nsplit, cus, s); break;
+                    case 16: launch_list<kKvPagedFp8, 16>(p, plan.nsplit, cus, s); break;
+                    case 8: launch_list<kKvPagedFp8, 8>(p, plan.nsplit, cus, s); break;
+                    default: launch_list<kKvPagedFp8, 0>(p, plan.nsplit, cus, s); break;
+                }
+            } else {
+                switch (seg) {
+                    case 32: launch_list<kKvPagedBf16, 32>(p, plan.nsplit, cus, s); break;
+                    case 16: launch_list<kKvPagedBf16, 16>(p, plan.nsplit, cus, s); break;
+                    case 8: launch_list<kKvPagedBf16, 8>(p, plan.nsplit, cus, s); break;
+                    case 4: launch_list<kKvPagedBf16, 4>(p, plan.nsplit, cus, s); break;
+                    default: launch_list<kKvPagedBf16, 0>(p, plan.nsplit, cus, s); break;
+                }
             }
-        } else {
-            switch (seg) {
-                case 32: launch_list<kKvPagedBf16, 32>(p, plan.nsplit, cus, s); break;
-                case 16: launch_list<kKvPagedBf16, 16>(p, plan.nsplit, cus, s); break;
-                case 8: launch_list<kKvPagedBf16, 8>(p, plan.nsplit, cus, s); break;
-                case 4: launch_list<kKvPagedBf16, 4>(p, plan.nsplit, cus, s); break;
-                default: launch_list<kKvPagedBf16, 0>(p, plan.nsplit, cus, s); break;
-            }
-        }
-        if (plan.nsplit > 1)
-            hipLaunchKernelGGL(decode_combine_kernel, dim3(p.hkv, p.batch), dim3(kDecThreads), 0, s, p);
+        };
+        run_ragged(p, work, pass1, s);
     }
     if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
     return FGQA_OK;

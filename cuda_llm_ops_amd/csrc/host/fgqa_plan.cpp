@@ -100,12 +100,29 @@ int plan_decode(const DecodeShape& a, int cus, DecodePlan* plan) {
         // tail.  Splits cost a partial write/read and a combine pass.
         if (cus <= 0) return FGQA_ERR_HIP;
         const int64_t items = (int64_t)(a.batch > 0 ? a.batch : 1) * a.num_kv_heads;
-        int64_t want = (items >= cus) ? 1 : ceil_div(4LL * cus, items);
-        const int64_t max_splits = ceil_div(S, kDecodeStepRound);
-        if (want > max_splits) want = max_splits;
-        if (want < 1) want = 1;
-        chunk = ceil_div(ceil_div(S, want), kDecodeStepRound) * kDecodeStepRound;
-        if (chunk > kDecodeMaxAutoChunk) chunk = kDecodeMaxAutoChunk;
+        chunk = kDecodeMaxAutoChunk;
+        if (items < cus) {
+            // Between 4096 tokens and 4 items per CU, the chunk with the
+            // fewest tokens in a row on one CU: rounds of the items over the
+            // CUs (one 8-wave workgroup of a head pair each, or two 4-wave
+            // ones) times the chunk and what an item costs beside it; the
+            // longer chunk of two that tie (fewer partials).  One 32768-token
+            // sequence, Hq = 64, Hkv = 8: 64 splits of 512 tokens (one round)
+            // 30.6 us, 128 of 256 (two rounds, the most splits) 33.8 us.
+            const int64_t want = ceil_div(4LL * cus, items);
+            int64_t lo = ceil_div(ceil_div(S, want), kDecodeStepRound) * kDecodeStepRound;
+            if (lo > kDecodeMaxAutoChunk) lo = kDecodeMaxAutoChunk;
+            int64_t best = -1;
+            for (int64_t c = kDecodeMaxAutoChunk; c >= lo; c -= kDecodeStepRound) {
+                if (c >= S + kDecodeStepRound) continue;
+                const int64_t rounds = ceil_div(ceil_div(S, c) * items, 2 * (int64_t)cus);
+                const int64_t cost = rounds * (c + kDecodeItemCost);
+                if (best < 0 || cost < best) {
+                    best = cost;
+                    chunk = c;
+                }
+            }
+        }
     }
     if (chunk < kDecodeStepRound) chunk = kDecodeStepRound;
     if (chunk > S) chunk = ceil_div(S, kDecodeStepRound) * kDecodeStepRound;
@@ -123,6 +140,18 @@ int plan_decode(const DecodeShape& a, int cus, DecodePlan* plan) {
     plan->part_o_bytes = round256(part_o);
     plan->part_ml_bytes = round256(part_ml);
     plan->ws_bytes = plan->part_o_bytes + plan->part_ml_bytes + (size_t)list;
+    plan->teams = 0;
+    plan->team_ml_off = plan->team_prefix_off = 0;
+    if (plan->list && a.split_tokens == 0 && a.num_kv_heads <= kDecodeItemSlots) {
+        // (the list's formula stays the least workspace, so that which calls
+        // fit a given scratch does not depend on how the batch is shared out)
+        plan->teams = kDecodeItemSlots / a.num_kv_heads;
+        const i128 rows = (i128)2 * plan->teams * a.num_q_heads;
+        plan->team_ml_off = round256(rows * kHeadDim * 4);
+        plan->team_prefix_off = plan->team_ml_off + round256(rows * 2 * 4);
+        const size_t need = plan->team_prefix_off + ((size_t)a.batch + 1) * 8;
+        if (need > plan->ws_bytes) plan->ws_bytes = need;
+    }
     return FGQA_OK;
 }
 

@@ -29,7 +29,14 @@ constexpr int kMaxTokens = 1 << 30;
 // ---------------------------------------------------------------- decode
 constexpr int kDecodeStepRound = 128;     // tokens of one pass of a decode workgroup's 4 waves
 constexpr int kDecodeMaxAutoChunk = 4096; // longest split the planner picks by itself
-constexpr int kDecodeRaggedChunk = 4096;  // split length for ragged batches (work-list mode)
+constexpr int kDecodeRaggedChunk = 4096;  // split length that bounds a ragged batch's workspace
+// 4-wave decode items the chip holds at once (two per CU on 256 CUs): a ragged
+// batch without a given split length is shared out evenly over teams of one
+// workgroup per kv head (pair) that together fill them.
+constexpr int kDecodeItemSlots = 512;
+// Cost of a decode item beyond its tokens (filling its load pipeline, the
+// waves' merge, its partial), in tokens a CU streams in that time.
+constexpr int kDecodeItemCost = 128;
 
 // Split plan inputs: the sizes alone (shared by the contiguous and paged entries).
 struct DecodeShape {
@@ -40,10 +47,15 @@ struct DecodeShape {
 struct DecodePlan {
     int chunk;            // tokens per split (a multiple of kDecodeStepRound)
     int nsplit;           // splits per sequence
-    bool list;            // ragged batch: a device-built work list of non-empty splits
+    bool list;            // ragged batch: teams, or (split length given) a device-built work list of non-empty splits
+    int teams;            // ragged batch without a given split length, at most kDecodeItemSlots kv heads: its
+                          // teams (else 0)
     size_t part_o_bytes;  // fp32 partial O of every split (nsplit > 1)
     size_t part_ml_bytes; // their (max, sum)
     size_t ws_bytes;      // the workspace: partials, then the list (1 + batch * nsplit int32)
+    // teams > 0: the workspace holds the partials of two items per team, their
+    // (max, sum) and the sequences' block prefix (batch + 1 int64) instead
+    size_t team_ml_off, team_prefix_off;
 };
 
 int validate_decode(const fgqa_decode_args* a);
