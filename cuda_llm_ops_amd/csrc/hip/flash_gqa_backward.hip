@@ -27,13 +27,9 @@
 //                      K/V tiles in LDS), dS^T on the VALU, dQ^T += K^T dS^T
 //                      (K read transposed).  bwd_dq_split_kernel: the same
 //                      unit with its key range split over two wave groups.
-//   bwd_dkdv_kernel    key-major: a workgroup owns a 128-key block of one KV
-//                      head (wave w: keys 32w..32w+31, K/V rows in registers)
-//                      and loops over (query head of its subset, 32-row query
-//                      block):  S = Q K^T, dP = dO V^T (Q/dO rows from LDS),
-//                      P and dS on the VALU (in place as bf16 A operands),
-//                      dV += P^T dO, dK += dS^T Q (dO/Q read transposed,
-//                      ds_read_b64_tr_b16).  dK/dV stay in registers (fp32).
+//   bwd_dkdv_kernel    key-major (flash_gqa_backward_dkdv.hip): a workgroup owns
+//                      a 128-key block of one KV head and loops over (query
+//                      head of its subset, 32-row query block).
 //   bwd_dkdv_reduce_kernel  only when a KV head's query heads are split over
 //                      several workgroups: sums their fp32 partial dK/dV.
 #include <math.h>
@@ -41,71 +37,11 @@
 
 #include <type_traits>
 
+#include "backward_common.h"
 #include "fgqa_device.h"
 #include "fgqa_internal.h"
 
 namespace fgqa {
-
-struct BwdParams {
-    const __bf16* q;
-    const __bf16* k;
-    const __bf16* v;
-    const __bf16* o;
-    const __bf16* dout;
-    const float* lse;
-    __bf16* dq;
-    __bf16* dk;
-    __bf16* dv;
-    int64_t q_sb, q_ss, q_sh;
-    int64_t k_sb, k_ss, k_sh;
-    int64_t v_sb, v_ss, v_sh;
-    int64_t o_sb, o_ss, o_sh;
-    int64_t do_sb, do_ss, do_sh;
-    int64_t dq_sb, dq_ss, dq_sh;
-    int64_t dk_sb, dk_ss, dk_sh;
-    int64_t dv_sb, dv_ss, dv_sh;
-    // workspace
-    float* rowstat;   // [2][B*Hq*Sq]: -lse*log2(e), then -delta*scale
-    float* dk_part;   // [n_hsplit][B, Hkv, Skv, D] fp32 partial sums (heads split), else null
-    float* dv_part;
-    int batch, sq, skv, hq, hkv, group, causal;
-    int window;       // > 0: sliding window (causal), row i uses keys (i - window, i]
-    // key-major (dK/dV) grid
-    int hs;           // query heads per workgroup
-    int n_hsplit;     // group / hs
-    int n_kvblocks;   // ceil(skv / 128)
-    int kv_streams;   // n_hsplit * hkv * batch
-    int n_qblocks32;  // ceil(sq / 32)
-    // query-major (dQ) grid, as the forward's
-    int hb;           // heads per 128-row unit
-    int n_hgroups;    // group / hb
-    int n_qunits;     // ceil(sq / (128 / hb))
-    int q_streams;    // n_hgroups * hkv * batch
-    float scale;
-    float scale_log2;   // scale * log2(e)
-};
-
-constexpr int kBwWaves = 4;
-constexpr int kBwThreads = kBwWaves * kWave;
-constexpr int kBwRowBytes = kHeadDim * 2;             // one Q / dO / K / V row
-constexpr int kBwHiRowBytes = 128;                    // dims 128..191 of a 192-wide Q / K row
-
-// ---- key-major kernel
-constexpr int kKvRing = 6;                            // operands read ahead in a step
-constexpr int kKvKeys = 128;                          // keys per workgroup
-constexpr int kKvRows = 32;                           // query rows per step
-constexpr int kKvTileBytes = kKvRows * kBwRowBytes;   // 8 KB: Q or dO of one step
-constexpr int kKvStatBytes = 2 * kKvRows * 4;         // -lse*log2e and -delta*scale of 32 rows
-// LDS: Q[3] | dO[3] | stats[3]
-constexpr int kKvQOff = 0;
-constexpr int kKvDoOff = 3 * kKvTileBytes;
-constexpr int kKvStatOff = 6 * kKvTileBytes;
-constexpr int kKvSmemBytes = kKvStatOff + 3 * kKvStatBytes;
-// MLA: the 128-byte parts of Q[3] follow
-constexpr int kKvQHiTileBytes = kKvRows * kBwHiRowBytes;   // 4 KB
-constexpr int kKvQHiOff = kKvSmemBytes;
-template <int kDk>
-constexpr int kv_smem_bytes() { return kDk > 128 ? kKvSmemBytes + 3 * kKvQHiTileBytes : kKvSmemBytes; }
 
 // ---- query-major kernel
 constexpr int kDqTile = 64;                           // keys per tile
@@ -117,77 +53,6 @@ constexpr int kDqKHiTileBytes = kDqTile * kBwHiRowBytes;   // 8 KB
 constexpr int kDqKHiOff = kDqSmemBytes;
 template <int kDk>
 constexpr int dq_smem_bytes() { return kDk > 128 ? kDqSmemBytes + 2 * kDqKHiTileBytes : kDqSmemBytes; }
-
-// Q, dO, K and V rows (256 B) sit in LDS with their 16-byte chunks permuted:
-// chunk c of row r goes to slot c ^ bw_swz(r).  bw_swz is a bijection on
-// r % 16 (16 consecutive rows read at the same chunk hit 16 different slots:
-// conflict-free b128 row reads) whose top two bits are r % 4 (4 consecutive
-// rows read over 4 consecutive chunks hit 4 disjoint slot groups:
-// conflict-free transposed reads).
-__device__ __forceinline__ int bw_swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
-
-__device__ __forceinline__ void bw_dma16(uint32_t lds_addr, uint32_t voffset, __amdgpu_buffer_rsrc_t rsrc) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :: "s"(lds_addr), "v"(voffset), "s"(rsrc) : "memory");
-}
-__device__ __forceinline__ void bw_dma4(uint32_t lds_addr, uint32_t voffset, __amdgpu_buffer_rsrc_t rsrc) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-                 :: "s"(lds_addr), "v"(voffset), "s"(rsrc) : "memory");
-}
-__device__ __forceinline__ void bw_wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// Byte offset, within a block of 16 swizzled 256-byte rows, that lane supplies
-// to a transposed read (ds_read_b64_tr_b16) so that the wave receives the
-// 32x32x16 MFMA operand  X[k = row][n = 32*cb + l32]  with the k order used
-// throughout: slots 0..3 of lane (l32, half g2) = rows 4*g2 + 0..3 (h8 = 0),
-// slots 4..7 = rows 8 + 4*g2 + 0..3 (h8 = 1).  Source lane (g2, gq, l16)
-// points at row 4*g2 + l16/4 + 8*h8, columns 32*cb + 16*gq + 4*(l16%4) .. +3.
-__device__ __forceinline__ int bw_tr_off(int lane, int cb, int h8) {
-    const int l16 = lane & 15, gq = (lane >> 4) & 1, g2 = lane >> 5;
-    const int r = 4 * g2 + (l16 >> 2) + 8 * h8;
-    const int c = 4 * cb + 2 * gq + ((l16 >> 1) & 1);
-    return r * kBwRowBytes + ((c ^ bw_swz(r)) << 4) + 8 * (l16 & 1);
-}
-
-// MLA (Q/K head dim 192, V/O 128): a 192-wide Q or K row is kept as a
-// 256-byte part (dims 0..127, laid out as above) and a 128-byte part (dims
-// 128..191) in a separate tile, whose chunk c of row r sits in slot
-// c ^ bw_swz_hi(r).  bw_swz_hi is a bijection on (r / 2) % 8: 16 consecutive
-// rows read at one chunk fall in 16 different 16-byte bank groups (rows of
-// either parity share none, 128-byte rows alternate halves of a 256-byte
-// bank line).  Its top bit is (r / 2) % 2: rows r and r + 2 read over 4
-// consecutive chunks land in different 4-chunk halves, so the transposed
-// reads are conflict-free too.
-__device__ __forceinline__ int bw_swz_hi(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
-// bw_tr_off for the 128-byte part (column block cb = 0, 1: dims 128 + 32cb ..)
-__device__ __forceinline__ int bw_tr_off_hi(int lane, int cb, int h8) {
-    const int l16 = lane & 15, gq = (lane >> 4) & 1, g2 = lane >> 5;
-    const int r = 4 * g2 + (l16 >> 2) + 8 * h8;
-    const int c = 4 * cb + 2 * gq + ((l16 >> 1) & 1);
-    return r * kBwHiRowBytes + ((c ^ bw_swz_hi(r)) << 4) + 8 * (l16 & 1);
-}
-template <int kDk>
-struct BwDims {
-    static_assert(kDk == 128 || kDk == 192, "Q/K head dim");
-    static constexpr bool kHi = kDk > 128;        // a 128-byte part per row
-    static constexpr int kRowBytes = kDk * 2;     // one Q / K row in HBM
-    static constexpr int kSteps = kDk / 16;       // MFMA k-steps of S over the Q/K dim
-    static constexpr int kDb = kDk / 32;          // 32-column blocks of dQ / dK
-};
-
-__device__ __forceinline__ bf16x8_t tr_pair(const unsigned char* base, int off0, int off1) {
-    const bf16x4_t lo = lds_read_tr16(reinterpret_cast<const __bf16*>(base + off0));
-    const bf16x4_t hi = lds_read_tr16(reinterpret_cast<const __bf16*>(base + off1));
-    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void bw_static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        bw_static_for<N, I + 1>(f);
-    }
-}
 
 // ---------------------------------------------------------------- row statistics
 // -lse*log2(e) and -delta*scale of one query row, delta = sum_d O[d] dO[d],
@@ -207,378 +72,6 @@ __device__ __forceinline__ float row_delta(const bf16x8_t (&oop)[8], const bf16x
         pair[kk] = xor_sum(acc, 32);
     }
     return ((pair[0] + pair[1]) + (pair[2] + pair[3])) + ((pair[4] + pair[5]) + (pair[6] + pair[7]));
-}
-
-// ---------------------------------------------------------------- dK / dV
-// Software pipelined one step ahead: step t runs
-//   phase A: S(t+1), dP(t+1) on the MFMA pipe  ||  P(t), dS(t) on the VALU
-//   phase B: dV += P(t)^T dO(t), dK += dS(t)^T Q(t) on the MFMA pipe
-// with Q/dO(t+2) streaming into the third LDS buffer meanwhile.
-// kSwa: sliding window (a separate instantiation, so the causal kernels carry
-// none of its work).  kAddMask: the mask enters as an additive -inf on S (any
-// nonzero scale); without it (scale 0, where -inf * 0 is not -inf) as a select
-// on P.
-template <bool kSwa, int kDk, bool kAddMask>
-__global__ __launch_bounds__(kBwThreads, 1) void bwd_dkdv_kernel(BwdParams p) {
-    using D = BwDims<kDk>;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int l32 = lane & 31;
-    const int l16 = lane & 15;
-    const int g2 = lane >> 5;
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
-
-    // Block -> (key block, head subset, kv head, batch).  Key blocks in
-    // ascending order: under the causal mask block 0 sees every query block,
-    // so the heaviest workgroups are dispatched first.
-    const int stream = blockIdx.x % p.kv_streams;
-    const int kb = blockIdx.x / p.kv_streams;
-    const int hsp = stream % p.n_hsplit;
-    const int kvh = (stream / p.n_hsplit) % p.hkv;
-    const int b = stream / (p.n_hsplit * p.hkv);
-    const int kv0 = kb * kKvKeys;
-    const int h0 = kvh * p.group + hsp * p.hs;
-
-    // K, V rows of this wave's keys as B operands of S = Q K^T, dP = dO V^T:
-    // lane (key l32, half g2), k-step ks holds elements 16ks + 8g2 .. +7.
-    // Keys >= skv read as zero.
-    const uint32_t kss = (uint32_t)(p.k_ss * 2);
-    const uint32_t vss = (uint32_t)(p.v_ss * 2);
-    const __amdgpu_buffer_rsrc_t krs =
-        make_rsrc(p.k + b * p.k_sb + kvh * p.k_sh, (uint32_t)(p.skv - 1) * kss + D::kRowBytes);
-    const __amdgpu_buffer_rsrc_t vrs =
-        make_rsrc(p.v + b * p.v_sb + kvh * p.v_sh, (uint32_t)(p.skv - 1) * vss + kBwRowBytes);
-    const int key = kv0 + 32 * wave + l32;   // this lane's key (column of S)
-    bf16x8_t kop[D::kSteps], vop[8];
-#pragma unroll
-    for (int ks = 0; ks < D::kSteps; ++ks)
-        kop[ks] = as_bf16x8(buf_load16(krs, (uint32_t)key * kss + (16 * ks + 8 * g2) * 2));
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
-        vop[ks] = as_bf16x8(buf_load16(vrs, (uint32_t)key * vss + (16 * ks + 8 * g2) * 2));
-
-    // step t: head h0 + t / per_head, query block qb0 + t % per_head
-    const int qb0 = p.causal ? min(kv0 / kKvRows, p.n_qblocks32) : 0;
-    // a window ends the key block's rows at its last key + window - 1
-    const int qb_end = kSwa ? min(p.n_qblocks32, (kv0 + kKvKeys + p.window - 2) / kKvRows + 1) : p.n_qblocks32;
-    const int per_head = max(0, qb_end - qb0);
-    const int n_iter = p.hs * per_head;
-
-    const uint32_t qss = (uint32_t)(p.q_ss * 2);
-    const uint32_t dss = (uint32_t)(p.do_ss * 2);
-    const int64_t rows_q = (int64_t)p.batch * p.hq * p.sq;
-    const __amdgpu_buffer_rsrc_t srs = make_rsrc(p.rowstat, (uint32_t)(2 * rows_q * 4));
-    // Q, dO rows of step t (wave w fetches rows 8w..8w+7 of each) and their
-    // statistics (wave 0) into buffer bi.  Rows >= sq read as zero.
-    // Steps are loaded in order, so the (head, query block) of the next load
-    // advances by one per call (no division per step).
-    int ld_h = h0, ld_qb = qb0;
-    int cur_qb = qb0;   // query block of the step being computed
-    auto issue = [&](int bi) {
-        const int hh = ld_h;
-        const int q0 = ld_qb * kKvRows;
-        if (++ld_qb == qb_end) {
-            ld_qb = qb0;
-            ++ld_h;
-        }
-        const __amdgpu_buffer_rsrc_t qrs =
-            make_rsrc(p.q + b * p.q_sb + hh * p.q_sh, (uint32_t)(p.sq - 1) * qss + D::kRowBytes);
-        const __amdgpu_buffer_rsrc_t drs =
-            make_rsrc(p.dout + b * p.do_sb + hh * p.do_sh, (uint32_t)(p.sq - 1) * dss + kBwRowBytes);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int r0 = 8 * wave + 4 * j;
-            const int r = r0 + (lane >> 4);
-            const int slot = (l16 ^ bw_swz(r)) << 4;
-            bw_dma16(lds_base + kKvQOff + bi * kKvTileBytes + r0 * kBwRowBytes, (uint32_t)(q0 + r) * qss + slot, qrs);
-            bw_dma16(lds_base + kKvDoOff + bi * kKvTileBytes + r0 * kBwRowBytes, (uint32_t)(q0 + r) * dss + slot, drs);
-        }
-        if constexpr (D::kHi) {
-            // dims 128..191 of rows 8w..8w+7: lane l fills slot l % 8 of row 8w + l / 8
-            const int r = 8 * wave + (lane >> 3);
-            const int c = (lane & 7) ^ bw_swz_hi(r);
-            bw_dma16(lds_base + kKvQHiOff + bi * kKvQHiTileBytes + 8 * wave * kBwHiRowBytes,
-                     (uint32_t)(q0 + r) * qss + kBwRowBytes + 16 * c, qrs);
-        }
-        if (wave == 0) {
-            const int r = q0 + l32;
-            const int64_t idx = ((int64_t)b * p.hq + hh) * p.sq + r + (g2 ? rows_q : 0);
-            const uint32_t off = (r < p.sq) ? (uint32_t)(idx * 4) : 0xFFFFFFF0u;   // out of range -> 0
-            bw_dma4(lds_base + kKvStatOff + bi * kKvStatBytes, off, srs);
-        }
-    };
-
-    f32x16_t dk_acc[D::kDb], dv_acc[4];
-#pragma unroll
-    for (int db = 0; db < D::kDb; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dk_acc[db][i] = 0.f;
-#pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dv_acc[db][i] = 0.f;
-
-    // transposed-read offsets into the Q / dO tiles
-    int trq[4][2], trq_hi[2][2];
-#pragma unroll
-    for (int db = 0; db < 4; ++db) {
-        trq[db][0] = bw_tr_off(lane, db, 0);
-        trq[db][1] = bw_tr_off(lane, db, 1);
-    }
-    if constexpr (D::kHi) {
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-            trq_hi[cb][0] = bw_tr_off_hi(lane, cb, 0);
-            trq_hi[cb][1] = bw_tr_off_hi(lane, cb, 1);
-        }
-    }
-    // b128 row-read offsets of the A operands of S and dP (row l32, chunk 2ks + g2)
-    int roff[8], roff_hi[4];
-    const int fl = bw_swz(l32);
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) roff[ks] = l32 * kBwRowBytes + (((2 * ks + g2) ^ fl) << 4);
-    if constexpr (D::kHi) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-            roff_hi[ks] = l32 * kBwHiRowBytes + (((2 * ks + g2) ^ bw_swz_hi(l32)) << 4);
-    }
-    const float c2 = p.scale_log2;
-    const float scale = p.scale;
-    // S = Q K^T and dP = dO V^T of the step in buffer bi: C[q][key], lane
-    // (key l32, half g2), register 4i + r <-> query row 8i + 4g2 + r
-    // Element (i, r) of a step's S block is query row q0 + 8i + 4g2 + r; it is
-    // masked (P = 0) when 8i + r < m, with m = key - q0 - 4g2 under the causal
-    // mask, and (window) when 8i + r > mx, mx = key + window - 1 - q0 - 4g2;
-    // steps past n_iter are fully masked.  Rows >= sq need no mask: their dO
-    // rows and -delta*scale read as zero, so P.dO and dS vanish; keys >= skv
-    // only reach their own dK/dV rows, which are never stored.
-    //
-    // kAddMask: the accumulator of a step's S starts at 0 or, on a step whose
-    // block the mask cuts (wave-uniform: the diagonal, the window's edge,
-    // padding), at ninf for each masked element, ninf = -inf times the sign of
-    // scale, so that S * scale * log2(e) is -inf and P = exp2(-inf) = +0 and
-    // dS = 0 * x, the values the select gives (for finite Q and K).  Only the
-    // first MFMA of S's chain differs between the two (its C operand: the
-    // literal 0, or the start values), and the softmax carries no
-    // per-element select: two VALU ops per element fewer.
-    const int wk0 = kv0 + 32 * wave;   // the wave's first key
-    const float ninf = c2 > 0.f ? -INFINITY : INFINITY;
-    auto is_cut = [&](int ts, int q0s) {
-        bool cut = ts >= n_iter || (p.causal && q0s < wk0 + 31);
-        if constexpr (kSwa) cut = cut || q0s + 31 > wk0 + p.window - 1;
-        return cut;
-    };
-    // the start values of a cut step's S block
-    auto bias = [&](int ts, int q0s) {
-        const int m = (ts < n_iter) ? (p.causal ? key - q0s - 4 * g2 : -64) : 64;
-        const int mx = key + p.window - 1 - q0s - 4 * g2;
-        f32x16_t b;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const bool vis = kSwa ? (8 * i + r >= m && 8 * i + r <= mx) : (8 * i + r >= m);
-                b[4 * i + r] = vis ? 0.f : ninf;
-            }
-        return b;
-    };
-    // S's first MFMA (k-step 0), with the mask's start values on cut steps
-    auto s_first = [&](const bf16x8_t& a, int ts, int q0s) -> f32x16_t {
-        f32x16_t z;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) z[i] = 0.f;
-        if (kAddMask && is_cut(ts, q0s)) return mfma32(a, kop[0], bias(ts, q0s));
-        return mfma32(a, kop[0], z);
-    };
-    auto sdp = [&](f32x16_t& s, f32x16_t& dp, auto bi_c) {
-        constexpr int bi = decltype(bi_c)::value;
-        const unsigned char* ql = smem + kKvQOff + bi * kKvTileBytes;
-        const unsigned char* dl = smem + kKvDoOff + bi * kKvTileBytes;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dp[i] = 0.f;
-        s = s_first(*reinterpret_cast<const bf16x8_t*>(ql + roff[0]), 0, qb0 * kKvRows);
-        dp = mfma32(*reinterpret_cast<const bf16x8_t*>(dl + roff[0]), vop[0], dp);
-#pragma unroll
-        for (int ks = 1; ks < 8; ++ks) {
-            s = mfma32(*reinterpret_cast<const bf16x8_t*>(ql + roff[ks]), kop[ks], s);
-            dp = mfma32(*reinterpret_cast<const bf16x8_t*>(dl + roff[ks]), vop[ks], dp);
-        }
-        if constexpr (D::kHi) {
-            const unsigned char* qh = smem + kKvQHiOff + bi * kKvQHiTileBytes;
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-                s = mfma32(*reinterpret_cast<const bf16x8_t*>(qh + roff_hi[ks]), kop[8 + ks], s);
-        }
-    };
-    // P = exp2(S*scale*log2e - lse*log2e), dS = P (dP - delta) scale, both as
-    // bf16 A operands (k-step ks = registers 8ks .. 8ks+7); without kAddMask
-    // the mask above is a select here.
-    bf16x8_t pop[2], dsop[2];
-    auto softmax = [&](const f32x16_t& s, const f32x16_t& dp, auto bi_c, int m, int mx) {
-        constexpr int bi = decltype(bi_c)::value;
-        const float* st = reinterpret_cast<const float*>(smem + kKvStatOff + bi * kKvStatBytes);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const f32x4_t nl = *reinterpret_cast<const f32x4_t*>(st + 8 * i + 4 * g2);
-            const f32x4_t nd = *reinterpret_cast<const f32x4_t*>(st + kKvRows + 8 * i + 4 * g2);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float pv = fast_exp2(__builtin_fmaf(s[4 * i + r], c2, nl[r]));
-                if constexpr (!kAddMask && kSwa)
-                    pv = (8 * i + r >= m && 8 * i + r <= mx) ? pv : 0.f;
-                else if constexpr (!kAddMask)
-                    pv = (8 * i + r >= m) ? pv : 0.f;
-                const float ds = pv * __builtin_fmaf(dp[4 * i + r], scale, nd[r]);
-                pop[i >> 1][(i & 1) * 4 + r] = (__bf16)pv;
-                dsop[i >> 1][(i & 1) * 4 + r] = (__bf16)ds;
-            }
-        }
-    };
-
-    // Triple-buffered Q/dO: step t reads buffers t%3 (dV/dK) and (t+1)%3
-    // (S/dP of the next step) while step t+2 lands in (t+2)%3, which step t-1
-    // finished with before the barrier that ended it.  The loop runs a
-    // multiple of 3 steps so that every buffer offset is a constant; steps
-    // past n_iter are fully masked (m = 64) and read buffers that hold zeros
-    // or an earlier step's rows, so they add exact zeros.  No branch touches
-    // the accumulators.
-    {
-        // zero the buffers first: a padded step may read one never loaded
-        const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-        for (int off = tid * 16; off < kv_smem_bytes<kDk>(); off += kBwThreads * 16)
-            *reinterpret_cast<f32x4_t*>(smem + off) = z;
-    }
-    __syncthreads();
-    if (n_iter > 0) issue(0);
-    if (n_iter > 1) issue(1);
-    bw_wait_vmem();
-    __syncthreads();
-
-    using C0 = std::integral_constant<int, 0>;
-    using C1 = std::integral_constant<int, 1>;
-    using C2 = std::integral_constant<int, 2>;
-    // step t: sc/dpc hold S/dP(t), sn/dpn receive S/dP(t+1); buffers BC = t%3,
-    // BN = (t+1)%3, BF = (t+2)%3
-    auto step = [&](f32x16_t& sc, f32x16_t& dpc, f32x16_t& sn, f32x16_t& dpn, int t, auto bc, auto bn, auto bf) {
-        if (t + 2 < n_iter) issue(decltype(bf)::value);
-        // query block of step t (advanced once per step, as the loads are)
-        const int q0 = cur_qb * kKvRows;
-        if (++cur_qb == qb_end) cur_qb = qb0;
-        [[maybe_unused]] const int m = (t < n_iter) ? (p.causal ? key - q0 - 4 * g2 : -64) : 64;
-        [[maybe_unused]] const int mx = key + p.window - 1 - q0 - 4 * g2;
-
-        // S/dP(t+1), then dV += P^T dO and dK += dS^T Q of step t (C[key][d],
-        // 4 column tiles of D; k-step ks takes query rows 16ks + 4g2 + 0..3
-        // and 16ks + 8 + 4g2 + 0..3, read transposed from the tiles), as one
-        // stream of operands read kKvRing MFMAs ahead into a ring of
-        // registers (6 ahead: 0.4 % faster than 4 at the 4096-token, 16-head
-        // shape, 1.5 % with the MLA head dims); P/dS(t) on the VALU between
-        // (the scheduler moves them up under the S/dP MFMAs).  Pinning the
-        // order with sched_group_barrier
-        // (reads kKvRing ahead, with or without the VALU spread over the S/dP
-        // MFMAs) was 5-17 % slower.
-        constexpr int BC = decltype(bc)::value, BN = decltype(bn)::value;
-        constexpr int kS = D::kHi ? 20 : 16;
-        constexpr int kOps = kS + (D::kHi ? 20 : 16);
-        constexpr int kR = kKvRing;
-        const unsigned char* qln = smem + kKvQOff + BN * kKvTileBytes;
-        const unsigned char* dln = smem + kKvDoOff + BN * kKvTileBytes;
-        const unsigned char* qlc = smem + kKvQOff + BC * kKvTileBytes;
-        const unsigned char* dlc = smem + kKvDoOff + BC * kKvTileBytes;
-        auto fetch = [&](auto ic) -> bf16x8_t {
-            constexpr int i = decltype(ic)::value;
-            if constexpr (i < 16) {
-                // S (i even) / dP (i odd) A operand, k-step i / 2
-                return *reinterpret_cast<const bf16x8_t*>((i % 2 == 0 ? qln : dln) + roff[i / 2]);
-            } else if constexpr (i < kS) {
-                const unsigned char* qh = smem + kKvQHiOff + BN * kKvQHiTileBytes;
-                return *reinterpret_cast<const bf16x8_t*>(qh + roff_hi[(i - 16) % 4]);
-            } else if constexpr (i < kS + 16) {
-                // dV (r even) / dK (r odd) B operand: k-step r / 8, column block (r / 2) % 4
-                constexpr int r = i - kS, ks = r / 8, db = (r / 2) % 4;
-                return tr_pair((r % 2 == 0 ? dlc : qlc) + ks * 16 * kBwRowBytes, trq[db % 4][0], trq[db % 4][1]);
-            } else {
-                constexpr int r = i - kS - 16, ks = r / 2, cb = r % 2;
-                const unsigned char* qh = smem + kKvQHiOff + BC * kKvQHiTileBytes + ks * 16 * kBwHiRowBytes;
-                return tr_pair(qh, trq_hi[cb % 2][0], trq_hi[cb % 2][1]);
-            }
-        };
-        bf16x8_t ring[kR];
-        bw_static_for<kR>([&](auto ic) { ring[decltype(ic)::value] = fetch(ic); });
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dpn[i] = 0.f;
-        // S(t+1)'s first MFMA ahead of the scheduled stream (cur_qb is now
-        // step t+1's block); its operand slot is refilled as op 0 would
-        sn = s_first(ring[0], t + 1, cur_qb * kKvRows);
-        ring[0] = fetch(std::integral_constant<int, kR>{});
-        auto op = [&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            const bf16x8_t a = ring[i % kR];
-            if constexpr (i == 0) {
-                (void)a;   // issued above
-            } else if constexpr (i < 16) {
-                if constexpr (i % 2 == 0) sn = mfma32(a, kop[i / 2], sn);
-                else dpn = mfma32(a, vop[i / 2], dpn);
-            } else if constexpr (i < kS) {
-                sn = mfma32(a, kop[8 + (i - 16) % 4], sn);
-            } else if constexpr (i < kS + 16) {
-                constexpr int r = i - kS, ks = r / 8, db = (r / 2) % 4;
-                if constexpr (r % 2 == 0) dv_acc[db] = mfma32(pop[ks], a, dv_acc[db]);
-                else dk_acc[db] = mfma32(dsop[ks], a, dk_acc[db]);
-            } else {
-                constexpr int r = i - kS - 16, ks = r / 2, cb = r % 2;
-                dk_acc[4 + cb % 2] = mfma32(dsop[ks], a, dk_acc[4 + cb % 2]);
-            }
-            if constexpr (i > 0 && i + kR < kOps) ring[i % kR] = fetch(std::integral_constant<int, i + kR>{});
-        };
-        // The scheduler's small-GEMM interleave (LLVM's IGLP strategy 0)
-        // issues the operand reads progressively further ahead of their
-        // MFMAs (up to 14 in flight) instead of just before each; without
-        // it most MFMAs waited on an LDS read (lgkmcnt 0 or 1).  Strategies
-        // 1-3 were slower.
-        __builtin_amdgcn_iglp_opt(0);
-        bw_static_for<kS>(op);
-        softmax(sc, dpc, bc, m, mx);
-        bw_static_for<kOps - kS>([&](auto ic) { op(std::integral_constant<int, kS + decltype(ic)::value>{}); });
-        bw_wait_vmem();
-        __syncthreads();
-    };
-    f32x16_t sa, dpa, sb, dpb, sx, dpx;
-    sdp(sa, dpa, C0{});
-    for (int t = 0; t < n_iter; t += 3) {
-        step(sa, dpa, sb, dpb, t, C0{}, C1{}, C2{});
-        step(sb, dpb, sx, dpx, t + 1, C1{}, C2{}, C0{});
-        step(sx, dpx, sa, dpa, t + 2, C2{}, C0{}, C1{});
-    }
-
-    // dK, dV of this wave's keys: C[key][d], lane (d = 32db + l32, half g2),
-    // register 4i + r <-> key 32w + 8i + 4g2 + r.  One workgroup per (key
-    // block, head subset): bf16 straight out, or an fp32 partial per subset.
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int j = kv0 + 32 * wave + 8 * i + 4 * g2 + r;
-            if (j >= p.skv) continue;
-            if (p.dk_part != nullptr) {
-                const int64_t row = (((int64_t)hsp * p.batch + b) * p.hkv + kvh) * p.skv + j;
-                float* dkr = p.dk_part + row * kDk + l32;
-                float* dvr = p.dv_part + row * kHeadDim + l32;
-#pragma unroll
-                for (int db = 0; db < D::kDb; ++db) dkr[32 * db] = dk_acc[db][4 * i + r];
-#pragma unroll
-                for (int db = 0; db < 4; ++db) dvr[32 * db] = dv_acc[db][4 * i + r];
-            } else {
-                __bf16* dkr = p.dk + b * p.dk_sb + (int64_t)j * p.dk_ss + kvh * p.dk_sh + l32;
-                __bf16* dvr = p.dv + b * p.dv_sb + (int64_t)j * p.dv_ss + kvh * p.dv_sh + l32;
-#pragma unroll
-                for (int db = 0; db < D::kDb; ++db) dkr[32 * db] = (__bf16)dk_acc[db][4 * i + r];
-#pragma unroll
-                for (int db = 0; db < 4; ++db) dvr[32 * db] = (__bf16)dv_acc[db][4 * i + r];
-            }
-        }
 }
 
 // Sum of the n_hsplit fp32 partials -> bf16 dK, dV.  16 lanes per key row:
@@ -665,7 +158,6 @@ __device__ __forceinline__ void dq_unit(const BwdParams& p, unsigned char* smem,
         doop[kk] = as_bf16x8(buf_load16(drs, (uint32_t)qrow * dss + (16 * kk + 8 * g2) * 2));
         oop[kk] = as_bf16x8(buf_load16(ors, (uint32_t)qrow * oss + (16 * kk + 8 * g2) * 2));
     }
-    const int64_t rows_q = (int64_t)p.batch * p.hq * p.sq;
     const int64_t ridx = ((int64_t)b * p.hq + h) * p.sq + qrow;
     const float nl = (qrow < p.sq) ? -p.lse[ridx] * kLog2e : 0.f;
     float nd = 0.f;   // set once O has arrived (after the first tile's loads are issued)
@@ -879,8 +371,7 @@ __device__ __forceinline__ void dq_unit(const BwdParams& p, unsigned char* smem,
     // the row's statistics, for this kernel's tiles and stored for dK/dV
     nd = (qrow < p.sq) ? -row_delta(oop, doop) * p.scale : 0.f;
     if (qrow < p.sq && g2 == 0) {
-        p.rowstat[ridx] = nl;
-        p.rowstat[rows_q + ridx] = nd;
+        *reinterpret_cast<f32x2_t*>(p.rowstat + 2 * ridx) = f32x2_t{nl, nd};
     }
     __syncthreads();
     using C0 = std::integral_constant<int, 0>;
@@ -973,7 +464,6 @@ __device__ __forceinline__ void dq_unit_pp(const BwdParams& p, unsigned char* sm
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) oop[kk] = as_bf16x8(buf_load16(ors, (uint32_t)qrow * oss + (16 * kk + 8 * g2) * 2));
     }
-    const int64_t rows_q = (int64_t)p.batch * p.hq * p.sq;
     const int64_t ridx = ((int64_t)b * p.hq + h) * p.sq + qrow;
     const float nl = (qrow < p.sq) ? -p.lse[ridx] * kLog2e : 0.f;
     float nd = 0.f;   // set once O has arrived (after the first tiles' loads are issued)
@@ -988,8 +478,7 @@ __device__ __forceinline__ void dq_unit_pp(const BwdParams& p, unsigned char* sm
         nd = (qrow < p.sq) ? -row_delta(oop, doop) * p.scale : 0.f;
         *nd_x = nd;
         if (qrow < p.sq && g2 == 0) {
-            p.rowstat[ridx] = nl;
-            p.rowstat[rows_q + ridx] = nd;
+            *reinterpret_cast<f32x2_t*>(p.rowstat + 2 * ridx) = f32x2_t{nl, nd};
         }
     };
     // group 1, after the barrier that follows stats(): the value is read and
@@ -1239,8 +728,6 @@ __global__ __launch_bounds__(2 * kBwThreads, 1) void bwd_dq_split_kernel(BwdPara
     dq_unit_pp<kSwa>(p, smem, qb, hg, kvh, b);
 }
 
-static_assert(kKvKeys == plan::kBackwardKvKeys, "keys per dK/dV workgroup");
-
 }  // namespace fgqa
 
 using namespace fgqa;
@@ -1384,9 +871,9 @@ int backward_launch(const fgqa_prefill_backward_args* a, hipStream_t s) {
     p.window = a->window_size;
     p.n_hsplit = pl.n_hsplit;
     p.hs = p.group / pl.n_hsplit;
-    p.n_kvblocks = (int)ceil_div(p.skv, kKvKeys);
+    p.n_kvblocks = (int)ceil_div(p.skv, plan::kBackwardKvKeys);
     p.kv_streams = pl.n_hsplit * p.hkv * p.batch;
-    p.n_qblocks32 = (int)ceil_div(p.sq, kKvRows);
+    p.n_qblocks32 = (int)ceil_div(p.sq, 32);
     p.hb = (p.group % 4 == 0) ? 4 : (p.group % 2 == 0) ? 2 : 1;
     p.n_hgroups = p.group / p.hb;
     p.n_qunits = (int)ceil_div(p.sq, 128 / p.hb);
@@ -1407,15 +894,9 @@ int backward_launch(const fgqa_prefill_backward_args* a, hipStream_t s) {
     const bool mla = a->head_dim == 192;
     const bool dq_split = a->dq_kernel == FGQA_KERNEL_AUTO ? (q_units < 4 * (int64_t)cus && !swa && !mla)
                                                            : a->dq_kernel == FGQA_KERNEL_SPLIT;
-    // the dK/dV kernel's mask: additive (-inf on S) unless the scale is 0
+    // the kernels' masks: additive (-inf on S) unless the scale is 0
     const int am = p.scale_log2 != 0.f ? 1 : 0;
-    // kernel table: [swa] of dK/dV ([additive mask] too), dQ, split dQ
-    const void* kv_fn[2][2] = {{reinterpret_cast<const void*>(bwd_dkdv_kernel<false, 128, false>),
-                                reinterpret_cast<const void*>(bwd_dkdv_kernel<false, 128, true>)},
-                               {reinterpret_cast<const void*>(bwd_dkdv_kernel<true, 128, false>),
-                                reinterpret_cast<const void*>(bwd_dkdv_kernel<true, 128, true>)}};
-    const void* kv192_fn[2] = {reinterpret_cast<const void*>(bwd_dkdv_kernel<false, 192, false>),
-                               reinterpret_cast<const void*>(bwd_dkdv_kernel<false, 192, true>)};
+    // kernel table: [swa][additive mask] of dQ, [swa] of split dQ
     const void* q_fn[2][2] = {{reinterpret_cast<const void*>(bwd_dq_kernel<false, 128, false>),
                                reinterpret_cast<const void*>(bwd_dq_kernel<false, 128, true>)},
                               {reinterpret_cast<const void*>(bwd_dq_kernel<true, 128, false>),
@@ -1424,12 +905,10 @@ int backward_launch(const fgqa_prefill_backward_args* a, hipStream_t s) {
                               reinterpret_cast<const void*>(bwd_dq_kernel<false, 192, true>)};
     const void* q2_fn[2] = {reinterpret_cast<const void*>(bwd_dq_split_kernel<false>),
                             reinterpret_cast<const void*>(bwd_dq_split_kernel<true>)};
-    // attribute slots 10..17 and 24..29: the backward kernels
+    // attribute slots 12..15, 17 and 27..29: the dQ kernels (dK/dV: launch_dkdv)
     if (mla) {
-        if ((st = set_kernel_smem_once(am ? 16 : 26, kv192_fn[am], kv_smem_bytes<192>())) != FGQA_OK) return st;
         if ((st = set_kernel_smem_once(am ? 17 : 29, q192_fn[am], dq_smem_bytes<192>())) != FGQA_OK) return st;
     } else {
-        if ((st = set_kernel_smem_once((am ? 10 : 24) + swa, kv_fn[swa][am], kKvSmemBytes)) != FGQA_OK) return st;
         if ((st = set_kernel_smem_once((am ? 12 : 27) + swa, q_fn[swa][am], kDqSmemBytes)) != FGQA_OK) return st;
         if ((st = set_kernel_smem_once(14 + swa, q2_fn[swa], kDqPpSmemBytes)) != FGQA_OK) return st;
     }
@@ -1443,12 +922,7 @@ int backward_launch(const fgqa_prefill_backward_args* a, hipStream_t s) {
         else if (q_units > 0)
             hipLaunchKernelGGL((bwd_dq_kernel<false, 192, false>), dim3((unsigned)q_units), dim3(kBwThreads),
                                dq_smem_bytes<192>(), s, p);
-        if (kv_units > 0 && am)
-            hipLaunchKernelGGL((bwd_dkdv_kernel<false, 192, true>), dim3((unsigned)kv_units), dim3(kBwThreads),
-                               kv_smem_bytes<192>(), s, p);
-        else if (kv_units > 0)
-            hipLaunchKernelGGL((bwd_dkdv_kernel<false, 192, false>), dim3((unsigned)kv_units), dim3(kBwThreads),
-                               kv_smem_bytes<192>(), s, p);
+        if (kv_units > 0 && (st = launch_dkdv(p, false, 192, am != 0, (unsigned)kv_units, s)) != FGQA_OK) return st;
         if (pl.n_hsplit > 1 && rows_kv > 0)
             hipLaunchKernelGGL(bwd_dkdv_reduce_kernel<192>, dim3((unsigned)ceil_div(rows_kv, 16)), dim3(256), 0, s,
                                p);
@@ -1469,13 +943,7 @@ int backward_launch(const fgqa_prefill_backward_args* a, hipStream_t s) {
         else if (am) hipLaunchKernelGGL((bwd_dq_kernel<false, 128, true>), g, t, kDqSmemBytes, s, p);
         else hipLaunchKernelGGL((bwd_dq_kernel<false, 128, false>), g, t, kDqSmemBytes, s, p);
     }
-    if (kv_units > 0) {
-        const dim3 g((unsigned)kv_units), t(kBwThreads);
-        if (swa && am) hipLaunchKernelGGL((bwd_dkdv_kernel<true, 128, true>), g, t, kKvSmemBytes, s, p);
-        else if (swa) hipLaunchKernelGGL((bwd_dkdv_kernel<true, 128, false>), g, t, kKvSmemBytes, s, p);
-        else if (am) hipLaunchKernelGGL((bwd_dkdv_kernel<false, 128, true>), g, t, kKvSmemBytes, s, p);
-        else hipLaunchKernelGGL((bwd_dkdv_kernel<false, 128, false>), g, t, kKvSmemBytes, s, p);
-    }
+    if (kv_units > 0 && (st = launch_dkdv(p, swa, 128, am != 0, (unsigned)kv_units, s)) != FGQA_OK) return st;
     if (pl.n_hsplit > 1 && rows_kv > 0)
         hipLaunchKernelGGL(bwd_dkdv_reduce_kernel<128>, dim3((unsigned)ceil_div(rows_kv, 16)), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
