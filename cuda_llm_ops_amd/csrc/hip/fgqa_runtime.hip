@@ -12,7 +12,7 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mutex;      // device properties and kernel attributes
 std::mutex g_ws_mutex;   // the library-owned workspaces
 int g_cu_count[kMaxDevices] = {0};
-constexpr int kMaxKernelSlots = 32;
+constexpr int kMaxKernelSlots = 40;
 bool g_smem_set[kMaxDevices][kMaxKernelSlots] = {};
 void* g_ws_ptr[kMaxDevices] = {nullptr};
 size_t g_ws_bytes[kMaxDevices] = {0};

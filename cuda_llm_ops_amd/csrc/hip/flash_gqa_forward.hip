@@ -71,57 +71,76 @@ namespace fgqa {
 
 constexpr int kPfWaves = 4;                            // waves per group (one unit's rows)
 constexpr int kPfThreads = kPfWaves * kWave;
-constexpr int kPfVRowBytes = kHeadDim * 2;             // one V row (V/O head dim 128)
-constexpr int kPfVTileBytes = kPfTile * kPfVRowBytes;  // 16 KB
 constexpr float kPfRescaleSlack = 8.f;                 // log2 units: P <= 2^8 between rescales
 // merge area of the split kernel: per wave, 64 O values + max + sum per lane
 constexpr int kPfMergeFloats = 66;
-// Q tile of a unit staged in LDS by the split kernel (head dim 128): 4 waves x
-// 32 rows x 256 bytes, after the two groups' tile buffers (2 x 64 KB + 32 KB =
-// the CU's 160 KB).
-constexpr int kPfQStageBytes = kPfWaves * 32 * kHeadDim * 2;
-// Wide kernel (head dim 128): both wave groups work on one set of tile
-// buffers (K0, K1, V0, V1: 64 KB), followed by the 256-row unit's Q tile
-// (64 KB, later its O tile) and one word that broadcasts the arrival count.
-// A split unit's partial result: 66 floats per lane (64 of O, max, sum) of
-// each of the 8 waves.
-constexpr int kPwTileBytes = 4 * kPfVTileBytes;
-constexpr int kPwQBytes = 2 * kPfQStageBytes;
-constexpr int kPwSmemBytes = kPwTileBytes + kPwQBytes + 16;   // + 3 words that broadcast counter reads
-// With the MLA head dim (192) the wide kernel loads Q straight into registers
-// (a 256-row Q tile does not fit beside the 80 KB of tiles) and stages O in
-// the tile buffers, idle after the loop.
-constexpr int pw_smem_bytes(int dk) { return dk == kHeadDim ? kPwSmemBytes : 2 * (64 * 384) + 2 * kPfVTileBytes + 16; }
 static_assert(kPfPartFloats == 2 * kPfWaves * kPfMergeFloats * kWave, "merge slot size");
 
-// Sizes that depend on the Q/K head dim kDk (128; 192 for MLA; 256, which
-// only the whole-range kernel is built for).
+// Sizes that depend on the Q/K head dim kDk (64, with V/O of 64 too, for both
+// head dims up to 64; 128; 192 for MLA; 256, which only the whole-range kernel
+// is built for).
 template <int kDk>
 struct PfDims {
-    static_assert(kDk == 128 || kDk == 192 || kDk == 256, "Q/K head dim");
+    static_assert(kDk == 64 || kDk == 128 || kDk == 192 || kDk == 256, "Q/K head dim");
+    static constexpr int kDv = kDk == 64 ? 64 : kHeadDim;             // V/O head dim
     static constexpr int kRowBytes = kDk * 2;                         // one K row
+    static constexpr int kVRowBytes = kDv * 2;                        // one V row
     static constexpr int kChunks = kDk / 8;                           // 16-byte chunks per K row
-    static constexpr int kKTileBytes = kPfTile * kRowBytes;           // 16, 24 or 32 KB
-    static constexpr int kGroupBytes = 2 * kKTileBytes + 2 * kPfVTileBytes;   // K0, K1, V0, V1
+    static constexpr int kVChunks = kDv / 8;                          // and per V row
+    static constexpr int kVb = kDv / 32;                              // 32-column blocks of O
+    static constexpr int kKTileBytes = kPfTile * kRowBytes;           // 8, 16, 24 or 32 KB
+    static constexpr int kVTileBytes = kPfTile * kVRowBytes;          // 8 or 16 KB
+    static constexpr int kGroupBytes = 2 * kKTileBytes + 2 * kVTileBytes;   // K0, K1, V0, V1
     static constexpr int kSteps = kDk / 16;                           // MFMA k-steps over the head dim
     static constexpr int kDmaK = kDk / 32;                            // K-tile DMA instructions per wave
+    static constexpr int kDmaV = kDv / 32;                            // and V-tile ones
+    // O tile of a group's 4 waves x 32 rows, and (head dims up to 128, where
+    // the two-group kernels stage Q in LDS) its Q tile, after the two groups'
+    // tile buffers (head dim 128: 2 x 64 KB + 32 KB = the CU's 160 KB)
+    static constexpr int kQStageBytes = kPfWaves * 32 * kVRowBytes;
+    // LDS of the wide kernel: both wave groups work on one set of tile buffers
+    // (K0, K1, V0, V1), followed by the 256-row unit's Q tile (later its O
+    // tile) and 3 words that broadcast counter reads.  With the MLA head dim
+    // (192) it loads Q straight into registers (a 256-row Q tile does not fit
+    // beside the 80 KB of tiles) and stages O in the tile buffers, idle after
+    // the loop.  A split unit's partial result: 66 floats per lane (64 of O,
+    // max, sum; head dim 64 uses 32 of the 64) of each of the 8 waves.
+    static constexpr int kWideWords = kGroupBytes + (kDk <= kHeadDim ? 2 * kQStageBytes : 0);
+    static constexpr int kWideSmemBytes = kWideWords + 16;
     // Per-lane K read offsets: k-steps kk and kk + kKoffRegs read chunks
     // 2 * kKoffRegs apart, which the swizzle keeps 32 * kKoffRegs bytes apart.
-    static constexpr int kKoffRegs = kDk == 192 ? 4 : 8;
+    static constexpr int kKoffRegs = kDk == 192 || kDk == 64 ? 4 : 8;
     // K swizzle: chunk c of row r sits in slot c ^ kswz(r).  16 consecutive
     // rows read at one chunk hit 16 distinct 16-byte bank groups: 256- and
     // 512-byte rows all start at bank 0 (XOR with r % 16, which keeps c inside
     // its aligned block of 16); 384-byte rows start at bank 0 or 32 by row
     // parity, so an XOR with (r / 2) % 8 (which keeps c inside its aligned
-    // block of 8) spreads each parity class over 8 groups.
-    static __device__ __forceinline__ int kswz(int r) { return kDk == 192 ? ((r >> 1) & 7) : (r & 15); }
-    static_assert(kPfWaves * kPfMergeFloats * kWave * 4 <= 2 * kGroupBytes, "merge area must fit in the tile buffers");
+    // block of 8) spreads each parity class over 8 groups; 128-byte rows (head
+    // dim 64) likewise, by a bijection on (r / 2) % 8 whose top bit is
+    // (r / 2) % 2, so that the transposed V reads of 4 rows x 4 chunks are free
+    // of conflicts too.
+    static __device__ __forceinline__ int kswz(int r) {
+        return kDk == 64 ? ((((r >> 1) & 1) << 2) | ((r >> 2) & 3)) : kDk == 192 ? ((r >> 1) & 7) : (r & 15);
+    }
+    static __device__ __forceinline__ int vswz(int r) { return kDk == 64 ? kswz(r) : 4 * (r & 3); }
+    static_assert(kDk == 64 || kPfWaves * kPfMergeFloats * kWave * 4 <= 2 * kGroupBytes,
+                  "merge area must fit in the tile buffers");
 };
+
+// Byte offset of 16-byte chunk c of a row of n valid chunks: past them (head
+// dims below 64, on the kernels built for 64) an offset no buffer resource here
+// reaches, so that the load returns zeros.
+template <int kDk>
+__device__ __forceinline__ uint32_t pf_chunk_off(uint32_t off, int c, int n) {
+    if constexpr (kDk == 64) return c < n ? off : 0x80000000u;
+    return off;
+}
 
 // LDS tiles hold unpadded rows whose 16-byte chunks are permuted (XOR
 // swizzle) so that both read patterns are free of bank conflicts:
 //   K: chunk c of row r sits in slot c ^ kswz(r)       (16 rows, one chunk each: b128 reads)
-//   V: chunk c of row r sits in slot c ^ 4*(r % 4)     (4 rows x 4 chunks: transposed b64 reads)
+//   V: chunk c of row r sits in slot c ^ vswz(r), 4*(r % 4) for 256-byte rows
+//                                                      (4 rows x 4 chunks: transposed b64 reads)
 // Tiles are filled by buffer_load ... lds (16 bytes per lane straight into
 // LDS): one instruction writes 1 KB, lane l taking the l-th 16-byte slot of
 // it, so each lane fetches the chunk that belongs in its slot.
@@ -139,8 +158,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                                         int b, PfSeg seg = PfSeg{0, 0, 0, nullptr, nullptr}) {
     using D = PfDims<kDk>;
     static_assert(!kWide || kGroups == 2, "wide units: two groups");
-    // wide: the tile buffers, then (head dim 128) the Q/O area, then 3 broadcast words
-    [[maybe_unused]] constexpr int kWWords = D::kGroupBytes + (kDk == kHeadDim ? kPwQBytes : 0);
+    [[maybe_unused]] constexpr int kWWords = D::kWideWords;   // wide: the 3 broadcast words
     // opaque in the split kernel: its loop over units recomputes what depends
     // on the thread index inside each unit instead of holding it in
     // registers across the loop
@@ -175,18 +193,20 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
     const int kv_hi = min(kv_end, (t_first + n_tiles) * kPfTile);
 
     // Q^T as the B operand: lane holds Q[q0w + l32][16*kk + 8*g2 .. +7]; rows >= sq read as 0.
-    // The split kernel (head dim 128) stages the unit's Q tile in LDS first
+    // The split kernel (head dims up to 128) stages the unit's Q tile in LDS first
     // (kStageQ below): a direct load puts 32 rows 4 KB apart (BSHD) into
     // one instruction, 32 bytes each, and both groups would load the same rows.
-    constexpr bool kStageQ = kGroups == 2 && kDk == kHeadDim;
+    constexpr bool kStageQ = kGroups == 2 && kDk <= kHeadDim;
+    // valid bytes and chunks of a Q/K and a V/O row (below 64: the rest reads as zeros)
+    const int dk8 = kDk == 64 ? p.dk8 : D::kChunks, dv8 = kDk == 64 ? p.dv8 : D::kVChunks;
     const uint32_t qss = (uint32_t)(p.q_ss * 2);
     const __amdgpu_buffer_rsrc_t qrs =
-        make_rsrc(p.q + b * p.q_sb + h * p.q_sh, (uint32_t)(p.sq - 1) * qss + D::kRowBytes);
+        make_rsrc(p.q + b * p.q_sb + h * p.q_sh, (uint32_t)(p.sq - 1) * qss + 16 * dk8);
     bf16x8_t qop[D::kSteps];
     if constexpr (!kStageQ) {
 #pragma unroll
         for (int kk = 0; kk < D::kSteps; ++kk) {
-            u32x4_t t = buf_load16(qrs, (uint32_t)qrow * qss + (kk * 16 + g2 * 8) * 2);
+            u32x4_t t = buf_load16(qrs, pf_chunk_off<kDk>((uint32_t)qrow * qss + (kk * 16 + g2 * 8) * 2, 2 * kk + g2, dk8));
             t ^= p.q_sign;
             qop[kk] = as_bf16x8(t);
         }
@@ -198,9 +218,9 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
     const uint32_t vss = (uint32_t)(p.v_ss * 2);
     const int kv_last = p.skv > 0 ? p.skv - 1 : 0;
     const __amdgpu_buffer_rsrc_t krs =
-        make_rsrc(p.k + b * p.k_sb + kvh * p.k_sh, (uint32_t)kv_last * kss + D::kRowBytes);
+        make_rsrc(p.k + b * p.k_sb + kvh * p.k_sh, (uint32_t)kv_last * kss + 16 * dk8);
     const __amdgpu_buffer_rsrc_t vrs =
-        make_rsrc(p.v + b * p.v_sb + kvh * p.v_sh, (uint32_t)kv_last * vss + kHeadDim * 2);
+        make_rsrc(p.v + b * p.v_sb + kvh * p.v_sh, (uint32_t)kv_last * vss + 16 * dv8);
     // K(t_first + j) -> K buffer kb (skipped when kb < 0), V(t_first + j) -> V buffer vb.
     // Written as inline asm so that the compiler does not treat every later
     // LDS read as dependent on these writes (it would wait for them to land
@@ -222,32 +242,34 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
     // Per-lane byte offsets of those chunks within a tile; the tile's start
     // goes in the scalar offset.
     int krow_dma[D::kDmaK];
-    uint32_t kcol_dma[D::kDmaK], koff_dma[D::kDmaK], voff_dma[4];
+    uint32_t kcol_dma[D::kDmaK], koff_dma[D::kDmaK], voff_dma[D::kDmaV];
 #pragma unroll
     for (int i = 0; i < D::kDmaK; ++i) {
         const int slot = 64 * (wave + 4 * i) + lane;
         const int r = slot / D::kChunks;
         krow_dma[i] = r;
-        kcol_dma[i] = (uint32_t)(((slot % D::kChunks) ^ D::kswz(r)) << 4);
-        koff_dma[i] = (uint32_t)r * kss + kcol_dma[i];
+        const int c = (slot % D::kChunks) ^ D::kswz(r);
+        kcol_dma[i] = pf_chunk_off<kDk>((uint32_t)c << 4, c, dk8);
+        koff_dma[i] = pf_chunk_off<kDk>((uint32_t)r * kss + ((uint32_t)c << 4), c, dk8);
     }
+    // chunk of the row V instruction i of this lane fetches, and the row
+    auto v_row = [&](int i) { return (64 * (wave + 4 * i) + lane) / D::kVChunks; };
+    auto v_chunk = [&](int i) { return (lane % D::kVChunks) ^ D::vswz(v_row(i)); };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = 4 * (wave + 4 * i) + (lane >> 4);
-        voff_dma[i] = (uint32_t)r * vss + ((l16 ^ (4 * (r & 3))) << 4);
-    }
+    for (int i = 0; i < D::kDmaV; ++i)
+        voff_dma[i] = pf_chunk_off<kDk>((uint32_t)v_row(i) * vss + ((uint32_t)v_chunk(i) << 4), v_chunk(i), dv8);
     // kb / vb: an int, or (split kernel loop) a std::integral_constant, so that
     // every LDS address folds into the instructions' offset fields
     auto issue_tile = [&](int j, auto kb, auto vb) {
         const int t0 = (t_first + j) * kPfTile;
         const uint32_t kdst = lds_base + kb * D::kKTileBytes + 1024 * wave;
-        const uint32_t vdst = lds_base + 2 * D::kKTileBytes + vb * kPfVTileBytes + 1024 * wave;
+        const uint32_t vdst = lds_base + 2 * D::kKTileBytes + vb * D::kVTileBytes + 1024 * wave;
         // K and V instructions interleaved, K first
         if (t0 + kPfTile - 1 <= kv_last) {   // whole tile in range
             static_for<D::kDmaK>([&](auto ic) {
                 constexpr int i = decltype(ic)::value;
                 if (kb >= 0) dma16(ic, kdst, koff_dma[i], (uint32_t)t0 * kss, krs);
-                if constexpr (i < 4)
+                if constexpr (i < D::kDmaV)
                     if (vb >= 0) dma16(ic, vdst, voff_dma[i], (uint32_t)t0 * vss, vrs);
             });
         } else {   // last tile: rows past the last key are clamped to it
@@ -255,12 +277,12 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                 constexpr int i = decltype(ic)::value;
                 if (kb >= 0) {
                     const uint32_t tok = (uint32_t)min(t0 + krow_dma[i], kv_last);
-                    dma16(ic, kdst, tok * kss + kcol_dma[i], 0u, krs);
+                    dma16(ic, kdst, kDk == 64 && kcol_dma[i] >= 0x80000000u ? kcol_dma[i] : tok * kss + kcol_dma[i], 0u,
+                          krs);
                 }
-                if (vb >= 0 && i < 4) {
-                    const int r = 4 * (wave + 4 * i) + (lane >> 4);
-                    const uint32_t tok = (uint32_t)min(t0 + r, kv_last);
-                    dma16(ic, vdst, tok * vss + ((l16 ^ (4 * (r & 3))) << 4), 0u, vrs);
+                if (vb >= 0 && i < D::kDmaV) {
+                    const uint32_t tok = (uint32_t)min(t0 + v_row(i), kv_last);
+                    dma16(ic, vdst, pf_chunk_off<kDk>(tok * vss + ((uint32_t)v_chunk(i) << 4), v_chunk(i), dv8), 0u, vrs);
                 }
             });
         }
@@ -297,9 +319,9 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
     float m_run = -INFINITY;   // running max (log2 units) of this lane's row
     float m_use = 0.f;         // m_run, or 0 while m_run is -inf
     float l_run = 0.f;         // this lane's share of the row sum
-    f32x16_t oacc[4];
+    f32x16_t oacc[D::kVb];
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < D::kVb; ++db)
 #pragma unroll
         for (int i = 0; i < 16; ++i) oacc[db][i] = 0.f;
 
@@ -357,7 +379,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
             const float alpha = fast_exp2(m_use - m_new_use);   // 0 on the first tile
             l_run *= alpha;
 #pragma unroll
-            for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+            for (int db = 0; db < D::kVb; ++db) oacc[db] *= alpha;
             m_run = m_new;
             m_use = m_new_use;
         }
@@ -401,33 +423,40 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
     // V reads below.  Lane i of a 16-lane group supplies row 16*kb + 4*g2 + i/4
     // (+8), columns 32*db + 16*((lane/16)%2) + 4*(i%4) .. +3, which is chunk
     // 4*db + 2*((lane/16)%2) + (i%4)/2, half i%2 of the swizzled row.
-    int voff[4];
+    // (128-byte rows: the swizzles of rows r and r + 8 differ, so the second
+    // read has an offset of its own.)
+    int voff[D::kVb], voff8[D::kVb];
     {
         const int q4 = l16 >> 2;
         const int dh = (lane >> 4) & 1;
+        const int r = 4 * g2 + q4;
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
-            voff[db] = (4 * g2 + q4) * kPfVRowBytes + ((4 * (db ^ q4) + 2 * dh + ((l16 >> 1) & 1)) << 4) + 8 * (l16 & 1);
+        for (int db = 0; db < D::kVb; ++db) {
+            const int c = 4 * db + 2 * dh + ((l16 >> 1) & 1);
+            voff[db] = r * D::kVRowBytes + ((c ^ D::vswz(r)) << 4) + 8 * (l16 & 1);
+            voff8[db] = kDk == 64 ? (r + 8) * D::kVRowBytes + ((c ^ D::vswz(r + 8)) << 4) + 8 * (l16 & 1)
+                                  : voff[db] + 8 * D::kVRowBytes;
+        }
     }
+    auto v_operand = [&](const unsigned char* vl, int kb, int db) -> bf16x8_t {
+        const unsigned char* base = vl + 16 * kb * D::kVRowBytes;
+        const bf16x4_t lo = lds_read_tr16(reinterpret_cast<const __bf16*>(base + voff[db]));
+        const bf16x4_t hi = lds_read_tr16(reinterpret_cast<const __bf16*>(base + voff8[db]));
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
     auto pv = [&](auto buf) {
-        const unsigned char* vl = smem + 2 * D::kKTileBytes + buf * kPfVTileBytes;
+        const unsigned char* vl = smem + 2 * D::kKTileBytes + buf * D::kVTileBytes;
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                const unsigned char* base = vl + 16 * kb * kPfVRowBytes + voff[db];
-                const bf16x4_t lo = lds_read_tr16(reinterpret_cast<const __bf16*>(base));
-                const bf16x4_t hi = lds_read_tr16(reinterpret_cast<const __bf16*>(base + 8 * kPfVRowBytes));
-                const bf16x8_t va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                oacc[db] = mfma32(va, pop[kb], oacc[db]);
-            }
+            for (int db = 0; db < D::kVb; ++db) oacc[db] = mfma32(v_operand(vl, kb, db), pop[kb], oacc[db]);
     };
 
     // this wave's direct LDS loads have landed (then a barrier publishes them)
     auto wait_vmem = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
     // every load of this wave but the newest n has landed (loads complete in
-    // order); n is a multiple of 4 up to 8 (the split kernel's K and V tiles
-    // at head dim 128 take 4 instructions per wave each)
+    // order); n is up to 8, rounded down to a multiple of 4 (the split kernel's
+    // K and V tiles take 4 instructions per wave each at head dim 128, 2 at 64)
     [[maybe_unused]] auto wait_vmem_but = [](int n) {
         if (n >= 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
         else if (n >= 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
@@ -449,14 +478,21 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
             if (tid == 0) __hip_atomic_store(seg.ctr + 1 + seg.slot, my_xcc1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    // Staged Q: wave slot w's 32 rows fill 8 KB at kPfQStageBytes/4 * w past
-    // the tile buffers, row r at 256*r with chunk c in slot c ^ (r % 16) (the
-    // K layout).  One load instruction fills 1 KB = 4 whole rows; the wave of
-    // slot w in group g issues instructions 4g .. 4g+3 of its slot's 8, so
-    // each row is fetched once for both groups.
+    // Staged Q: wave slot w's 32 rows fill 8 KB (head dim 64: 4 KB) at
+    // kQStageBytes/4 * w past the tile buffers, row r at kRowBytes*r with chunk c
+    // in slot c ^ kswz(r) (the K layout).  One load instruction fills 1 KB = 4 (8)
+    // whole rows; the wave of slot w in group g issues its half of its slot's
+    // instructions, so each row is fetched once for both groups.
     [[maybe_unused]] const uint32_t q_lds =
-        kWide ? lds_base + kPwTileBytes + wave_wg * (kPfQStageBytes / kPfWaves)
-              : lds_base + (2 - grp) * D::kGroupBytes + wave * (kPfQStageBytes / kPfWaves);
+        kWide ? lds_base + D::kGroupBytes + wave_wg * (D::kQStageBytes / kPfWaves)
+              : lds_base + (2 - grp) * D::kGroupBytes + wave * (D::kQStageBytes / kPfWaves);
+    // instruction i of the wave's Q rows: row and byte offset of this lane's chunk
+    [[maybe_unused]] auto q_voff = [&](int i) {
+        const int slot = 64 * i + lane;
+        const int r = slot / D::kChunks;
+        const int c = (slot % D::kChunks) ^ D::kswz(r);
+        return pf_chunk_off<kDk>((uint32_t)(q0w + r) * qss + ((uint32_t)c << 4), c, dk8);
+    };
     if constexpr (kWide) {
         // a wide unit's waves have rows of their own: each loads its 8 KB
         // (head dim 192: Q came straight into registers above)
@@ -466,12 +502,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                 asm volatile("s_add_u32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                              :: "s"(base), "v"(voffset), "s"(rsrc), "i"(kOff) : "memory", "scc");
             };
-            static_for<8>([&](auto ic) {
-                const int slot = 64 * decltype(ic)::value + lane;
-                const int r = slot >> 4;
-                const uint32_t voff = (uint32_t)(q0w + r) * qss + ((uint32_t)((slot & 15) ^ (r & 15)) << 4);
-                dmaq(ic, q_lds, voff, qrs);
-            });
+            static_for<D::kRowBytes / 32>([&](auto ic) { dmaq(ic, q_lds, q_voff(decltype(ic)::value), qrs); });
         }
         // group 0 loads K(0); group 1 loads V(0) and K(1), awaited by the end
         // of its S(0) phase (group 0's first MFMA phase comes after that)
@@ -481,7 +512,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
         } else {
             if (n_tiles > 0) issue_tile(0, -1, 0);
             if (n_tiles > 1) issue_tile(1, 1, -1);
-            wait_vmem_but((n_tiles > 0 ? 4 : 0) + (n_tiles > 1 ? D::kDmaK : 0));
+            wait_vmem_but((n_tiles > 0 ? D::kDmaV : 0) + (n_tiles > 1 ? D::kDmaK : 0));
         }
     } else if constexpr (kStageQ) {
         auto dmaq = [](auto ic, uint32_t base, uint32_t voffset, __amdgpu_buffer_rsrc_t rsrc) {
@@ -489,22 +520,19 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
             asm volatile("s_add_u32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                          :: "s"(base), "v"(voffset), "s"(rsrc), "i"(kOff) : "memory", "scc");
         };
-        static_for<4>([&](auto ic) {
-            const int slot = 64 * (4 * grp + decltype(ic)::value) + lane;
-            const int r = slot >> 4;
-            const uint32_t voff = (uint32_t)(q0w + r) * qss + ((uint32_t)((slot & 15) ^ (r & 15)) << 4);
-            dmaq(ic, q_lds + grp * 4096, voff, qrs);
+        constexpr int kHalf = D::kRowBytes / 64;   // a group's share of the instructions
+        static_for<kHalf>([&](auto ic) {
+            dmaq(ic, q_lds + grp * kHalf * 1024, q_voff(kHalf * grp + decltype(ic)::value), qrs);
         });
     }
     if constexpr (kWide) {
     } else if constexpr (kStageQ) {
         // the first barrier needs Q and K(0) only: V(0) and K(1) are waited
         // for by the first softmax phase
-        static_assert(D::kDmaK == 4, "wait_vmem_but counts 4 loads per tile");
         if (n_tiles > 0) issue_tile(0, 0, -1);
         if (n_tiles > 0) issue_tile(0, -1, 0);
         if (n_tiles > 1) issue_tile(1, 1, -1);
-        wait_vmem_but((n_tiles > 0 ? 4 : 0) + (n_tiles > 1 ? 4 : 0));
+        wait_vmem_but((n_tiles > 0 ? D::kDmaV : 0) + (n_tiles > 1 ? D::kDmaK : 0));
     } else {
         if (n_tiles > 0) issue_tile(0, 0, 0);
         if (n_tiles > 1) issue_tile(1, 1, -1);
@@ -513,12 +541,12 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
     __syncthreads();
     if constexpr (kStageQ) {
         const unsigned char* ql = reinterpret_cast<const unsigned char*>(smem_all) +
-                                  (kWide ? kPwTileBytes + wave_wg * (kPfQStageBytes / kPfWaves)
-                                         : 2 * D::kGroupBytes + wave * (kPfQStageBytes / kPfWaves)) +
+                                  (kWide ? D::kGroupBytes + wave_wg * (D::kQStageBytes / kPfWaves)
+                                         : 2 * D::kGroupBytes + wave * (D::kQStageBytes / kPfWaves)) +
                                   l32 * D::kRowBytes;
 #pragma unroll
         for (int kk = 0; kk < D::kSteps; ++kk) {
-            u32x4_t t = *reinterpret_cast<const u32x4_t*>(ql + (((2 * kk + g2) ^ (l32 & 15)) << 4));
+            u32x4_t t = *reinterpret_cast<const u32x4_t*>(ql + (((2 * kk + g2) ^ D::kswz(l32)) << 4));
             t ^= p.q_sign;
             qop[kk] = as_bf16x8(t);
         }
@@ -553,10 +581,10 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
         // V reads run 3 MFMAs ahead of their use
         __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);       // DS reads
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        for (int i = 0; i < 4 * D::kVb; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);   // VALU
-            if (i < 13) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // DS reads
+            __builtin_amdgcn_sched_group_barrier(0x002, 8 / D::kVb, 0);   // VALU
+            if (i < 4 * D::kVb - 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // DS reads
         }
         update_max(tmax);
         wait_vmem();
@@ -622,7 +650,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                 }
                 if (j + 2 < n_tiles) {
                     issue_tile(j + 2, CN{}, CV{});
-                    n_new += 4;
+                    n_new += D::kDmaV;
                 }
             }
             mask(s, j + 1);
@@ -659,12 +687,13 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
         auto mphase = [&](auto with_qk, int j, auto par) {
             constexpr int kA = decltype(with_qk)::value ? 2 * D::kSteps : 0;
             constexpr int P = decltype(par)::value;
-            constexpr int kOps = kA + 16;
+            constexpr int kPv = 4 * D::kVb;
+            constexpr int kOps = kA + kPv;
             (void)j;
             const unsigned char* kl = smem + (1 - P) * D::kKTileBytes;
-            const unsigned char* vl = smem + 2 * D::kKTileBytes + P * kPfVTileBytes;
+            const unsigned char* vl = smem + 2 * D::kKTileBytes + P * D::kVTileBytes;
             // operand i: K operand (kk, tb) = (i / 2, i % 2) for i < kA, else V
-            // operand (kb, db) = ((i - kA) / 4, (i - kA) % 4)
+            // operand (kb, db) = ((i - kA) / kVb, (i - kA) % kVb)
             auto fetch = [&](auto ic) -> bf16x8_t {
                 constexpr int i = decltype(ic)::value;
                 if constexpr (i < kA) {
@@ -672,11 +701,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                     const int off = tb * 32 * D::kRowBytes + koff[kk % D::kKoffRegs] + (kk / D::kKoffRegs) * (D::kKoffRegs * 32);
                     return *reinterpret_cast<const bf16x8_t*>(kl + off);
                 } else {
-                    constexpr int kb = (i - kA) / 4, db = (i - kA) % 4;
-                    const unsigned char* base = vl + 16 * kb * kPfVRowBytes + voff[db];
-                    const bf16x4_t lo = lds_read_tr16(reinterpret_cast<const __bf16*>(base));
-                    const bf16x4_t hi = lds_read_tr16(reinterpret_cast<const __bf16*>(base + 8 * kPfVRowBytes));
-                    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                    return v_operand(vl, (i - kA) / D::kVb, (i - kA) % D::kVb);
                 }
             };
             bf16x8_t ring[4];
@@ -693,7 +718,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                 if constexpr (i < kA) {
                     s[i % 2] = mfma32(a, qop[i / 2], s[i % 2]);
                 } else {
-                    constexpr int kb = (i - kA) / 4, db = (i - kA) % 4;
+                    constexpr int kb = (i - kA) / D::kVb, db = (i - kA) % D::kVb;
                     oacc[db] = mfma32(a, pop[kb], oacc[db]);
                 }
                 if constexpr (i + 4 < kOps) ring[i % 4] = fetch(std::integral_constant<int, i + 4>{});
@@ -714,9 +739,9 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                 __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
+            for (int i = 0; i < kPv; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                if (i < 12) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                if (i < kPv - 4) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             }
             // all of the phase's MFMAs before its barrier (the scheduler would
             // otherwise sink the last ones into the softmax phase)
@@ -796,7 +821,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                 const bool near = word[1] == my_xcc1;   // the reader shares this XCD's L2
                 f32x4_t* o4 = reinterpret_cast<f32x4_t*>(own) + lane;
 #pragma unroll
-                for (int db = 0; db < 4; ++db)
+                for (int db = 0; db < D::kVb; ++db)
 #pragma unroll
                     for (int i4 = 0; i4 < 4; ++i4)
                         o4[(db * 4 + i4) * kWave] = f32x4_t{oacc[db][4 * i4], oacc[db][4 * i4 + 1],
@@ -834,7 +859,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
             const float aB = fast_exp2(mB - mu);
             const f32x4_t* r4 = reinterpret_cast<const f32x4_t*>(other) + lane;
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < D::kVb; ++db)
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4) {
                     const f32x4_t ot = r4[(db * 4 + i4) * kWave];
@@ -850,34 +875,36 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
             m_use = mu;
         }
     } else if constexpr (kGroups == 2 && kStageQ) {
-        // Head dim 128: each group keeps O columns 64*grp .. +63 (blocks
-        // 2*grp, 2*grp + 1) and hands the other half, with its max and sum, to
+        // Head dims up to 128: each group keeps half of O's columns (head dim
+        // 128: 64*grp .. +63, blocks 2*grp, 2*grp + 1) and hands the other half, with its max and sum, to
         // the same wave slot of the other group through its own tile
-        // buffers (idle since the loop's last barrier): 8 blocks of [lane][4]
+        // buffers (idle since the loop's last barrier): 8 (or 4) blocks of [lane][4]
         // floats, then [lane] max and [lane] sum.  Both groups then merge and
         // store their half, so neither waits for the other to store all of O.
         // Both merge in one form, group 0's terms first, so the two halves of
         // a row share bit-identical max, sum and weights.
-        float* mine = reinterpret_cast<float*>(smem_all + grp * D::kGroupBytes) + wave * 34 * kWave;
-        const float* theirs = reinterpret_cast<const float*>(smem_all + (1 - grp) * D::kGroupBytes) + wave * 34 * kWave;
+        constexpr int kHb = D::kVb / 2;               // blocks of a half
+        constexpr int kHv = kHb * 16;                 // its values per lane
+        float* mine = reinterpret_cast<float*>(smem_all + grp * D::kGroupBytes) + wave * (kHv + 2) * kWave;
+        const float* theirs = reinterpret_cast<const float*>(smem_all + (1 - grp) * D::kGroupBytes) + wave * (kHv + 2) * kWave;
         f32x4_t* mw = reinterpret_cast<f32x4_t*>(mine) + lane;
         const f32x4_t* mr = reinterpret_cast<const f32x4_t*>(theirs) + lane;
         auto handoff = [&](auto od) {
             constexpr int o = decltype(od)::value;
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
+            for (int k = 0; k < kHb; ++k)
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4)
                     mw[(k * 4 + i4) * kWave] = f32x4_t{oacc[o + k][4 * i4], oacc[o + k][4 * i4 + 1],
                                                        oacc[o + k][4 * i4 + 2], oacc[o + k][4 * i4 + 3]};
         };
-        if (grp == 0) handoff(std::integral_constant<int, 2>{});
+        if (grp == 0) handoff(std::integral_constant<int, kHb>{});
         else handoff(std::integral_constant<int, 0>{});
-        mine[32 * kWave + lane] = m_run;
-        mine[33 * kWave + lane] = l_run;
+        mine[kHv * kWave + lane] = m_run;
+        mine[(kHv + 1) * kWave + lane] = l_run;
         __syncthreads();
-        const float m_o = theirs[32 * kWave + lane];
-        const float l_o = theirs[33 * kWave + lane];
+        const float m_o = theirs[kHv * kWave + lane];
+        const float l_o = theirs[(kHv + 1) * kWave + lane];
         const float mA = grp == 0 ? m_run : m_o, lA = grp == 0 ? l_run : l_o;   // group 0's
         const float mB = grp == 0 ? m_o : m_run, lB = grp == 0 ? l_o : l_run;   // group 1's
         const float m = fmaxf(mA, mB);
@@ -887,7 +914,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
         auto merge_half = [&](auto kd) {
             constexpr int o = decltype(kd)::value;
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
+            for (int k = 0; k < kHb; ++k)
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4) {
                     const f32x4_t other = mr[(k * 4 + i4) * kWave];
@@ -900,7 +927,7 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
                 }
         };
         if (grp == 0) merge_half(std::integral_constant<int, 0>{});
-        else merge_half(std::integral_constant<int, 2>{});
+        else merge_half(std::integral_constant<int, kHb>{});
         l_run = __builtin_fmaf(lA, aA, lB * aB);
         m_run = m;
         m_use = mu;
@@ -950,34 +977,36 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
     const float denom = (l_run > 0.f && has_sink) ? l_run + sink * fast_exp2(-m_use) : l_run;
     const float inv = (l_run > 0.f) ? 1.f / denom : 0.f;
     if constexpr (kGroups == 2 && kStageQ && !kWide) {
-        // this group's 64 columns of the wave's 32 rows go out through 4 KB of
-        // the (idle) Q area: 8-byte pieces into 128-byte half rows, chunk c of
-        // row r in slot c ^ (r % 8), then 8 half rows per store instruction
-        unsigned char* ol = smem_all + 2 * D::kGroupBytes + (grp * kPfWaves + wave) * 4096;
+        // this group's half of the columns (64; head dim 64: 32) of the wave's
+        // 32 rows go out through 4 KB (2 KB) of the (idle) Q area: 8-byte
+        // pieces into 128-byte (64-byte) half rows, chunk c of row r in slot
+        // c ^ (r % 8) (% 4), then 8 (16) half rows per store instruction
+        constexpr int kHb = D::kVb / 2, kHc = 4 * kHb, kHBytes = kHc * 16;
+        unsigned char* ol = smem_all + 2 * D::kGroupBytes + (grp * kPfWaves + wave) * 32 * kHBytes;
         auto stage = [&](auto kd) {
             constexpr int o = decltype(kd)::value;
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
+            for (int k = 0; k < kHb; ++k)
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4) {
                     bf16x4_t w;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) w[e] = (__bf16)(oacc[o + k][i4 * 4 + e] * inv);
-                    *reinterpret_cast<bf16x4_t*>(ol + l32 * 128 + (((4 * k + i4) ^ (l32 & 7)) << 4) + g2 * 8) = w;
+                    *reinterpret_cast<bf16x4_t*>(ol + l32 * kHBytes + (((4 * k + i4) ^ (l32 & (kHc - 1))) << 4) + g2 * 8) = w;
                 }
         };
         if (grp == 0) stage(std::integral_constant<int, 0>{});
-        else stage(std::integral_constant<int, 2>{});
+        else stage(std::integral_constant<int, kHb>{});
         // this wave's LDS writes complete before its reads (no other wave uses the area)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 8 * i + (lane >> 3);
-            const int cc = lane & 7;
-            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ol + r * 128 + ((cc ^ (r & 7)) << 4));
-            if (q0w + r < p.sq) {
+        for (int i = 0; i < 32 * kHBytes / 1024; ++i) {
+            const int r = (64 * i + lane) / kHc;
+            const int cc = lane % kHc;
+            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ol + r * kHBytes + ((cc ^ (r & (kHc - 1))) << 4));
+            if (q0w + r < p.sq && (kDk != 64 || kHc * grp + cc < dv8)) {
                 __bf16* orow = p.o + b * p.o_sb + (int64_t)(q0w + r) * p.o_ss + h * p.o_sh;
-                *reinterpret_cast<u32x4_t*>(orow + 64 * grp + 8 * cc) = v;
+                *reinterpret_cast<u32x4_t*>(orow + 8 * (kHc * grp + cc)) = v;
             }
         }
         if (grp == 1) return;   // group 0 writes the LSE
@@ -991,27 +1020,29 @@ __device__ __forceinline__ void pf_unit(const PrefillParams& p, unsigned char* s
         // give each store 32 rows 16 bytes each).
         static_assert(kGroups == 1 || kStageQ || kPfWaves * kPfMergeFloats * kWave * 4 <= D::kGroupBytes,
                       "O staging in group 1's buffers must not overlap the merge area");
-        unsigned char* ol = kWide ? smem_all + (kStageQ ? kPwTileBytes : 0) + wave_wg * (kPfQStageBytes / kPfWaves)
+        unsigned char* ol = kWide ? smem_all + (kStageQ ? D::kGroupBytes : 0) + wave_wg * (D::kQStageBytes / kPfWaves)
                                   : smem_all + (kGroups == 1 ? 0 : kStageQ ? 2 : 1) * D::kGroupBytes +
-                                        wave * (kPfQStageBytes / kPfWaves);
+                                        wave * (D::kQStageBytes / kPfWaves);
+        constexpr int kC = D::kVChunks;
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
+        for (int db = 0; db < D::kVb; ++db)
 #pragma unroll
             for (int i4 = 0; i4 < 4; ++i4) {
                 bf16x4_t w;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) w[e] = (__bf16)(oacc[db][i4 * 4 + e] * inv);
-                *reinterpret_cast<bf16x4_t*>(ol + l32 * kPfVRowBytes + (((4 * db + i4) ^ (l32 & 15)) << 4) + g2 * 8) = w;
+                *reinterpret_cast<bf16x4_t*>(ol + l32 * D::kVRowBytes + (((4 * db + i4) ^ (l32 & (kC - 1))) << 4) + g2 * 8) = w;
             }
         // this wave's LDS writes complete before its reads (no other wave uses the area)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int r = 4 * i + (lane >> 4);
-            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ol + r * kPfVRowBytes + (l16 << 4));
-            if (q0w + r < p.sq) {
+        for (int i = 0; i < 32 * kC / 64; ++i) {
+            const int r = (64 * i + lane) / kC;
+            const int cl = lane % kC, c = cl ^ (r & (kC - 1));
+            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ol + r * D::kVRowBytes + (cl << 4));
+            if (q0w + r < p.sq && (kDk != 64 || c < dv8)) {
                 __bf16* orow = p.o + b * p.o_sb + (int64_t)(q0w + r) * p.o_ss + h * p.o_sh;
-                *reinterpret_cast<u32x4_t*>(orow + ((l16 ^ (r & 15)) << 3)) = v;
+                *reinterpret_cast<u32x4_t*>(orow + (c << 3)) = v;
             }
         }
     }
@@ -1237,8 +1268,10 @@ namespace {
 // The launches of a validated (128, 128) or MLA call.
 int prefill_launch(const fgqa_prefill_args* a, hipStream_t s);
 
-// Head dims the kernels are not built for (plan::prefill_padded): pad, run
-// the built kernels on the copies (once per 128 columns of V), unpad O.  The
+// Head dims the kernels are not built for (plan::prefill_padded).  Both up to
+// 64 and aligned (plan::prefill_native64): the kernels built for 64, on the
+// tensors themselves (the workspace bytes asked for stay those of the copies).
+// Else: pad, run the built kernels on the copies (once per 128 columns of V), unpad O.  The
 // copies live in the caller's workspace after the merge scratch, or with
 // none in the library's cached buffer (the merge scratch then being the
 // library's per-device one).
@@ -1251,7 +1284,9 @@ int prefill_padded_launch(const fgqa_prefill_args* a, hipStream_t s) {
     std::unique_lock<std::mutex> lock;
     unsigned char* base = nullptr;   // the copies: base + L.q .. base + L.total
     unsigned char* ws = static_cast<unsigned char*>(a->workspace);
+    const bool native = plan::prefill_native64(a);
     if (ws == nullptr && a->workspace_bytes == 0) {
+        if (native) return prefill_launch(a, s);
         lock = workspace_lock();
         int st = FGQA_OK;
         unsigned char* buf = static_cast<unsigned char*>(internal_workspace(L.total - L.q, &st));
@@ -1267,6 +1302,7 @@ int prefill_padded_launch(const fgqa_prefill_args* a, hipStream_t s) {
             pa.workspace = ws;
             pa.workspace_bytes = merge;
         }
+        if (native) return prefill_launch(a, s);
     }
     __bf16* qp = reinterpret_cast<__bf16*>(base + L.q);
     __bf16* kp = reinterpret_cast<__bf16*>(base + L.k);
@@ -1340,6 +1376,15 @@ extern "C" int fgqa_prefill_bf16(const fgqa_prefill_args* a, void* stream) {
 namespace fgqa {
 namespace {
 
+// One of the 256-row kernels, on grid workgroups of 8 waves.
+template <int kDk>
+int launch_wide(void (*fn)(PrefillParams), int slot, dim3 grid, const PrefillParams& p, hipStream_t s) {
+    const int sm = PfDims<kDk>::kWideSmemBytes;
+    if (const int e = set_kernel_smem_once(slot, reinterpret_cast<const void*>(fn), sm); e != FGQA_OK) return e;
+    hipLaunchKernelGGL(fn, grid, dim3(2 * kPfThreads), sm, s, p);
+    return hipGetLastError() == hipSuccess ? FGQA_OK : FGQA_ERR_HIP;
+}
+
 int prefill_launch(const fgqa_prefill_args* a, hipStream_t s) {
     PrefillParams p;
     p.q = static_cast<const __bf16*>(a->q);
@@ -1378,6 +1423,8 @@ int prefill_launch(const fgqa_prefill_args* a, hipStream_t s) {
     p.q_sign = (a->scale < 0.f) ? 0x80008000u : 0u;
     p.window = a->window_size;
     p.sink = a->sink;
+    p.dk8 = a->head_dim / 8;
+    p.dv8 = (a->head_dim_v == 0 ? a->head_dim : a->head_dim_v) / 8;
     p.wide_bias = 0;
     p.wide_part = nullptr;
     p.wide_ctr = nullptr;
@@ -1402,6 +1449,7 @@ int prefill_launch(const fgqa_prefill_args* a, hipStream_t s) {
     }
     const bool swa = p.window > 0 || p.sink != nullptr;
     const bool mla = a->head_dim == 192;
+    const bool d64 = a->head_dim <= 64;   // (both head dims, aligned: plan::prefill_native64)
     const bool split = choice == FGQA_KERNEL_SPLIT;
     if (a->head_dim == 256) {
         // Q/K head dim 256: the whole-range kernel (the plan refuses the
@@ -1429,59 +1477,44 @@ int prefill_launch(const fgqa_prefill_args* a, hipStream_t s) {
         if (choice == FGQA_KERNEL_TALL) return launch_prefill_tall(p, tall_on_pairs(a, cus), cus, s);
         if (!wide_on_pairs(a, cus)) {
             // more pairs than one per two CUs: whole units on a persistent grid
-            // attribute slots 7, 8, 9: the persistent wide kernels (plain, window, MLA)
-            const int slot = mla ? 9 : swa ? 8 : 7;
-            const void* pfn = mla   ? reinterpret_cast<const void*>(prefill_wide_persistent_kernel<false, 192>)
-                              : swa ? reinterpret_cast<const void*>(prefill_wide_persistent_kernel<true, kHeadDim>)
-                                    : reinterpret_cast<const void*>(prefill_wide_persistent_kernel<false, kHeadDim>);
-            const int sm = pw_smem_bytes(a->head_dim);
-            if (const int e = set_kernel_smem_once(slot, pfn, sm); e != FGQA_OK) return e;
+            // attribute slots 7, 8, 9, 32, 33: the persistent wide kernels
             const int64_t units_w = (int64_t)p.n_qblocks * p.n_streams;
             const dim3 grid((unsigned)(units_w < cus ? units_w : cus));
-            if (mla) hipLaunchKernelGGL((prefill_wide_persistent_kernel<false, 192>), grid, dim3(2 * kPfThreads), sm, s, p);
-            else if (swa) hipLaunchKernelGGL((prefill_wide_persistent_kernel<true, kHeadDim>), grid, dim3(2 * kPfThreads), sm, s, p);
-            else hipLaunchKernelGGL((prefill_wide_persistent_kernel<false, kHeadDim>), grid, dim3(2 * kPfThreads), sm, s, p);
-            if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
-            return FGQA_OK;
+            if (mla) return launch_wide<192>(prefill_wide_persistent_kernel<false, 192>, 9, grid, p, s);
+            if (d64)
+                return swa ? launch_wide<64>(prefill_wide_persistent_kernel<true, 64>, 33, grid, p, s)
+                           : launch_wide<64>(prefill_wide_persistent_kernel<false, 64>, 32, grid, p, s);
+            return swa ? launch_wide<128>(prefill_wide_persistent_kernel<true, 128>, 8, grid, p, s)
+                       : launch_wide<128>(prefill_wide_persistent_kernel<false, 128>, 7, grid, p, s);
         }
-        // attribute slots 5, 6: the wide kernels
-        // attribute slots 5, 6, 18: the wide kernels (plain, window, MLA)
-        const int wslot = mla ? 18 : swa ? 6 : 5;
-        const void* wfn = mla   ? reinterpret_cast<const void*>(prefill_wide_kernel<false, 192>)
-                          : swa ? reinterpret_cast<const void*>(prefill_wide_kernel<true, kHeadDim>)
-                                : reinterpret_cast<const void*>(prefill_wide_kernel<false, kHeadDim>);
-        const int wsm = pw_smem_bytes(a->head_dim);
-        if (const int e = set_kernel_smem_once(wslot, wfn, wsm); e != FGQA_OK) return e;
+        // attribute slots 5, 6, 18, 34, 35: the wide kernels
         // blocks w and w + 8 of each 16 run one pair
         const dim3 grid((unsigned)(16 * ceil_div(wide_pairs(a), 8)));
-        if (mla) hipLaunchKernelGGL((prefill_wide_kernel<false, 192>), grid, dim3(2 * kPfThreads), wsm, s, p);
-        else if (swa) hipLaunchKernelGGL((prefill_wide_kernel<true, kHeadDim>), grid, dim3(2 * kPfThreads), wsm, s, p);
-        else hipLaunchKernelGGL((prefill_wide_kernel<false, kHeadDim>), grid, dim3(2 * kPfThreads), wsm, s, p);
-        if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
-        return FGQA_OK;
+        if (mla) return launch_wide<192>(prefill_wide_kernel<false, 192>, 18, grid, p, s);
+        if (d64)
+            return swa ? launch_wide<64>(prefill_wide_kernel<true, 64>, 35, grid, p, s)
+                       : launch_wide<64>(prefill_wide_kernel<false, 64>, 34, grid, p, s);
+        return swa ? launch_wide<128>(prefill_wide_kernel<true, 128>, 6, grid, p, s)
+                   : launch_wide<128>(prefill_wide_kernel<false, 128>, 5, grid, p, s);
     }
 
-    const int group_bytes = mla ? PfDims<192>::kGroupBytes : PfDims<128>::kGroupBytes;
-    // the split kernel with head dim 128 also stages the Q tile in LDS
-    const int smem_bytes = (split ? 2 : 1) * group_bytes + (split && !mla ? kPfQStageBytes : 0);
-    // kernel table: plain, window / sink, split, MLA, MLA split
-    const int which = mla ? (split ? 4 : 3) : (split ? 2 : (swa ? 1 : 0));
-    const void* fns[5] = {reinterpret_cast<const void*>(prefill_kernel<false, 128>),
-                          reinterpret_cast<const void*>(prefill_kernel<true, 128>),
-                          reinterpret_cast<const void*>(prefill_split_kernel<128>),
-                          reinterpret_cast<const void*>(prefill_kernel<false, 192>),
-                          reinterpret_cast<const void*>(prefill_split_kernel<192>)};
-    // attribute slots 0..4: the prefill kernels
-    if (const int e = set_kernel_smem_once(which, fns[which], smem_bytes); e != FGQA_OK) return e;
+    const int group_bytes = mla ? PfDims<192>::kGroupBytes : d64 ? PfDims<64>::kGroupBytes : PfDims<128>::kGroupBytes;
+    const int q_bytes = mla ? 0 : d64 ? PfDims<64>::kQStageBytes : PfDims<128>::kQStageBytes;
+    // the split kernel with head dims up to 128 also stages the Q tile in LDS
+    const int smem_bytes = (split ? 2 : 1) * group_bytes + (split ? q_bytes : 0);
+    // kernel table: plain, window / sink, split, MLA, MLA split, head dim 64's plain, window / sink, split
+    const int which = d64 ? (split ? 7 : (swa ? 6 : 5)) : mla ? (split ? 4 : 3) : (split ? 2 : (swa ? 1 : 0));
+    void (*const fns[8])(PrefillParams) = {
+        prefill_kernel<false, 128>, prefill_kernel<true, 128>, prefill_split_kernel<128>, prefill_kernel<false, 192>,
+        prefill_split_kernel<192>,  prefill_kernel<false, 64>, prefill_kernel<true, 64>,  prefill_split_kernel<64>};
+    // attribute slots 0..4 and 36..38: the prefill kernels
+    if (const int e = set_kernel_smem_once(which < 5 ? which : 31 + which, reinterpret_cast<const void*>(fns[which]),
+                                           smem_bytes);
+        e != FGQA_OK)
+        return e;
     // the split kernel is persistent: at most one workgroup per CU
     const dim3 grid((unsigned)(split && units > cus ? cus : units));
-    switch (which) {
-        case 0: hipLaunchKernelGGL((prefill_kernel<false, 128>), grid, dim3(kPfThreads), smem_bytes, s, p); break;
-        case 1: hipLaunchKernelGGL((prefill_kernel<true, 128>), grid, dim3(kPfThreads), smem_bytes, s, p); break;
-        case 2: hipLaunchKernelGGL(prefill_split_kernel<128>, grid, dim3(2 * kPfThreads), smem_bytes, s, p); break;
-        case 3: hipLaunchKernelGGL((prefill_kernel<false, 192>), grid, dim3(kPfThreads), smem_bytes, s, p); break;
-        default: hipLaunchKernelGGL(prefill_split_kernel<192>, grid, dim3(2 * kPfThreads), smem_bytes, s, p); break;
-    }
+    hipLaunchKernelGGL(fns[which], grid, dim3(split ? 2 * kPfThreads : kPfThreads), smem_bytes, s, p);
     if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
     return FGQA_OK;
 }

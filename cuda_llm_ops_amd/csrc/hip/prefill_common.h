@@ -34,6 +34,7 @@ struct PrefillParams {
     uint32_t q_sign;    // 0x80008000 when scale < 0 (Q is negated on load), else 0
     int window;         // > 0: sliding window, row i sees keys [i - window + 1, i] (causal)
     const float* sink;  // nullable [Hq]: added to the softmax denominator as sink * exp(-max)
+    int dk8, dv8;       // head dims up to 64: 16-byte chunks of a Q/K and of a V/O row
     // 256-row kernels whose unit pairs split a unit over two workgroups: tiles
     // a pair's heavy unit keeps beyond half the pair's tiles on its first
     // workgroup, and the partial-result slots and arrival counters of the

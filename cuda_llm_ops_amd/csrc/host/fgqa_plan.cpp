@@ -221,6 +221,16 @@ bool prefill_padded(const fgqa_prefill_args* a) {
     return a->head_dim > 0 && dv > 0 && a->head_dim <= 256 && dv <= 256 && !native_head_dims(a->head_dim, dv);
 }
 
+bool prefill_native64(const fgqa_prefill_args* a) {
+    const int dv = head_dim_v_of(a);
+    if (!prefill_padded(a) || a->head_dim > 64 || dv > 64 || (a->head_dim & 7) || (dv & 7)) return false;
+    if (a->kernel == FGQA_KERNEL_TALL) return false;
+    if (!aligned16(a->q) || !aligned16(a->k) || !aligned16(a->v) || !aligned16(a->o)) return false;
+    for (int i = 0; i < 3; ++i)
+        if ((a->q_stride[i] & 7) || (a->k_stride[i] & 7) || (a->v_stride[i] & 7) || (a->o_stride[i] & 7)) return false;
+    return true;
+}
+
 int padded_dk(const fgqa_prefill_args* a) {
     return a->head_dim <= kHeadDim ? kHeadDim : a->head_dim == 192 ? 192 : 256;
 }

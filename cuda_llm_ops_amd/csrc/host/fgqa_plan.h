@@ -91,6 +91,13 @@ int validate_prefill(const fgqa_prefill_args* a);
 // Triton kernels pad their head-dim blocks to a power of two the same way,
 // src/python/Triton/flash_gqa_kernel.py:266-269, 80-94.)
 bool prefill_padded(const fgqa_prefill_args* a);
+// A padded call that runs on the tensors themselves, on the kernels built for
+// head dim 64: both head dims up to 64 and multiples of 8, 16-byte aligned
+// pointers and strides in multiples of 8 (what those kernels' 16-byte accesses
+// need), and a kernel shape built for 64 (all but the tall one).  Columns past
+// the head dims read as zeros and are not written.  Same kernel shape, and the
+// same bits, as on the copies.
+bool prefill_native64(const fgqa_prefill_args* a);
 int padded_dk(const fgqa_prefill_args* a);
 int padded_dv(const fgqa_prefill_args* a);
 // The call on the copies (head dims padded_dk() and 128, V and O rows of
