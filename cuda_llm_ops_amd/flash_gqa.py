@@ -25,6 +25,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import operator
 
 import torch
 
@@ -58,12 +59,20 @@ __all__ = [
 ]
 
 
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
+def _ptr(t: torch.Tensor | None) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+# The raw handle of the current device's current stream.  torch's own accessors
+# build a Stream object for it (2.8 us a call against 0.2).
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+_get_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _get_device is None or _get_raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _get_raw_stream(_get_device())
 
 
 def _require_cuda(*ts: torch.Tensor) -> None:
@@ -74,9 +83,13 @@ def _require_cuda(*ts: torch.Tensor) -> None:
 
 def _kernel_ready(t: torch.Tensor) -> bool:
     """Head dim contiguous, 16-byte aligned base, strides multiple of 8 elements."""
-    if t.stride(-1) != 1 or t.data_ptr() % 16 != 0:
+    st = t.stride()
+    if st[-1] != 1 or t.data_ptr() & 15:
         return False
-    return all(s % 8 == 0 for s in t.stride()[:-1])
+    for s in st[:-1]:
+        if s & 7:
+            return False
+    return True
 
 
 def _prep(t: torch.Tensor) -> torch.Tensor:
@@ -87,21 +100,14 @@ def _prep(t: torch.Tensor) -> torch.Tensor:
 def _decode_args(q, k, v, o, scale, seqlens, lse, split_tokens, workspace) -> _lib.DecodeArgs:
     B, Hq, D = q.shape
     _, S, Hkv, _ = k.shape
-    a = _lib.DecodeArgs()
-    a.q, a.k, a.v, a.o = _ptr(q), _ptr(k), _ptr(v), _ptr(o)
-    a.lse = _ptr(lse)
-    a.seqlens = _ptr(seqlens)
-    a.batch, a.max_seqlen, a.num_q_heads, a.num_kv_heads, a.head_dim = B, S, Hq, Hkv, D
-    a.scale = float(scale)
-    a.q_stride[:] = [q.stride(0), q.stride(1)]
-    a.k_stride[:] = [k.stride(0), k.stride(1), k.stride(2)]
-    a.v_stride[:] = [v.stride(0), v.stride(1), v.stride(2)]
-    a.o_stride[:] = [o.stride(0), o.stride(1)]
-    a.split_tokens = int(split_tokens)
-    if workspace is not None:
-        a.workspace = workspace.data_ptr()
-        a.workspace_bytes = workspace.numel() * workspace.element_size()
-    return a
+    return _lib.pack_decode(
+        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(seqlens), B, S, Hq, Hkv, D, float(scale),
+        *q.stride()[:2], *k.stride()[:3], *v.stride()[:3], *o.stride()[:2], int(split_tokens), *_workspace(workspace))
+
+
+def _workspace(workspace):
+    """The workspace fields: its address and bytes, or none."""
+    return (0, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size())
 
 
 def decode_workspace_bytes(batch, max_seqlen, num_q_heads, num_kv_heads, head_dim=128, split_tokens=0,
@@ -164,7 +170,7 @@ def decode_flash_gqa_bshd(q, k, v, scale=None, out=None, seqlens=None, lse=None,
     Returns ``out`` (bf16 [B, Hq, D]).
     """
     a, out, _keep = _decode_prepare(q, k, v, scale, out, seqlens, lse, split_tokens, workspace)
-    _lib.check(_lib.lib().fgqa_decode_bf16(ctypes.byref(a), ctypes.c_void_p(_stream())), "fgqa_decode_bf16")
+    _lib.check(_lib.lib().fgqa_decode_bf16(ctypes.byref(a), _stream()), "fgqa_decode_bf16")
     return out
 
 
@@ -183,7 +189,7 @@ class PreparedLaunch:
         self._where = where
 
     def __call__(self):
-        st = self._fn(self._ref, ctypes.c_void_p(_stream()))
+        st = self._fn(self._ref, _stream())
         if st != _lib.FGQA_OK:
             raise _lib.FgqaError(st, self._where)
         return self.out
@@ -205,23 +211,11 @@ def _paged_args(q, kc, vc, block_table, seqlens, o, lse, scale, k_scale, v_scale
                 split_tokens, workspace):
     B, Hq, D = q.shape
     num_pages, page_size, Hkv, _ = kc.shape
-    a = _lib.PagedDecodeArgs()
-    a.q, a.k_cache, a.v_cache, a.o, a.lse = _ptr(q), _ptr(kc), _ptr(vc), _ptr(o), _ptr(lse)
-    a.block_table, a.seqlens = _ptr(block_table), _ptr(seqlens)
-    a.batch, a.max_seqlen, a.num_q_heads, a.num_kv_heads, a.head_dim = B, max_seqlen, Hq, Hkv, D
-    a.page_size, a.num_pages = page_size, num_pages
-    a.kv_dtype = _PAGED_DTYPES[kc.dtype]
-    a.scale, a.k_scale, a.v_scale = float(scale), float(k_scale), float(v_scale)
-    a.q_stride[:] = [q.stride(0), q.stride(1)]
-    a.o_stride[:] = [o.stride(0), o.stride(1)]
-    a.k_stride[:] = [kc.stride(0), kc.stride(1), kc.stride(2)]
-    a.v_stride[:] = [vc.stride(0), vc.stride(1), vc.stride(2)]
-    a.block_table_stride = block_table.stride(0) if block_table.dim() == 2 else 0
-    a.split_tokens = int(split_tokens)
-    if workspace is not None:
-        a.workspace = workspace.data_ptr()
-        a.workspace_bytes = workspace.numel() * workspace.element_size()
-    return a
+    return _lib.pack_paged(
+        _ptr(q), _ptr(kc), _ptr(vc), _ptr(o), _ptr(lse), _ptr(block_table), _ptr(seqlens), B, max_seqlen, Hq, Hkv, D,
+        page_size, num_pages, _PAGED_DTYPES[kc.dtype], float(scale), float(k_scale), float(v_scale),
+        *q.stride()[:2], *o.stride()[:2], *kc.stride()[:3], *vc.stride()[:3],
+        block_table.stride(0) if block_table.dim() == 2 else 0, int(split_tokens), *_workspace(workspace))
 
 
 def paged_decode_workspace_bytes(batch, max_seqlen, num_q_heads, num_kv_heads, page_size, head_dim=128,
@@ -290,7 +284,7 @@ def decode_flash_gqa_paged(q, k_cache, v_cache, block_table, seqlens, scale=None
     """
     a, out, _keep = _paged_prepare(q, k_cache, v_cache, block_table, seqlens, scale, k_scale, v_scale, out,
                                    lse, max_seqlen, split_tokens, workspace)
-    _lib.check(_lib.lib().fgqa_decode_paged(ctypes.byref(a), ctypes.c_void_p(_stream())), "fgqa_decode_paged")
+    _lib.check(_lib.lib().fgqa_decode_paged(ctypes.byref(a), _stream()), "fgqa_decode_paged")
     return out
 
 
@@ -340,46 +334,35 @@ def launch_decode_flash_gqa_bf16_kernel(q, k, v, out=None):
 
 
 # --------------------------------------------------------------------------- prefill
+# {batch, sequence, head} strides of a 4-D tensor's strides in each layout
+_SBH = {"bshd": operator.itemgetter(0, 1, 2), "bhsd": operator.itemgetter(0, 2, 1)}
+_KERNELS = {"auto": _lib.FGQA_KERNEL_AUTO, "whole": _lib.FGQA_KERNEL_WHOLE, "split": _lib.FGQA_KERNEL_SPLIT,
+            "wide": _lib.FGQA_KERNEL_WIDE, "tall": _lib.FGQA_KERNEL_TALL}
+
+
 def _kernel_choice(kernel) -> int:
     """'auto' / 'whole' / 'split' (or the FGQA_KERNEL_* value) -> the C ABI value."""
-    names = {"auto": _lib.FGQA_KERNEL_AUTO, "whole": _lib.FGQA_KERNEL_WHOLE, "split": _lib.FGQA_KERNEL_SPLIT,
-             "wide": _lib.FGQA_KERNEL_WIDE, "tall": _lib.FGQA_KERNEL_TALL}
     if isinstance(kernel, str):
-        if kernel not in names:
-            raise ValueError(f"kernel must be one of {sorted(names)}")
-        return names[kernel]
+        if kernel not in _KERNELS:
+            raise ValueError(f"kernel must be one of {sorted(_KERNELS)}")
+        return _KERNELS[kernel]
     return int(kernel)
 
 
 def _prefill_args(q, k, v, o, lse, scale, causal, layout, window_size=0, sink=None,
                   kernel="auto") -> _lib.PrefillArgs:
     """C ABI argument block for q/k/v/o 4-D in `layout` ('bshd' or 'bhsd')."""
-    def sbh(t):
-        if layout == "bshd":
-            return [t.stride(0), t.stride(1), t.stride(2)]
-        return [t.stride(0), t.stride(2), t.stride(1)]
-
     if layout == "bshd":
         B, Sq, Hq, D = q.shape
         _, Skv, Hkv, _ = k.shape
     else:
         B, Hq, Sq, D = q.shape
         _, Hkv, Skv, _ = k.shape
-    a = _lib.PrefillArgs()
-    a.q, a.k, a.v, a.o, a.lse = _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse)
-    a.batch, a.seqlen_q, a.seqlen_kv = B, Sq, Skv
-    a.num_q_heads, a.num_kv_heads, a.head_dim = Hq, Hkv, D
-    a.head_dim_v = v.shape[3]
-    a.causal = 1 if causal else 0
-    a.scale = float(scale)
-    a.q_stride[:] = sbh(q)
-    a.k_stride[:] = sbh(k)
-    a.v_stride[:] = sbh(v)
-    a.o_stride[:] = sbh(o)
-    a.window_size = int(window_size)
-    a.sink = _ptr(sink)
-    a.kernel = _kernel_choice(kernel)
-    return a
+    sbh = _SBH[layout]
+    return _lib.pack_prefill(
+        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), B, Sq, Skv, Hq, Hkv, D, 1 if causal else 0, float(scale),
+        *sbh(q.stride()), *sbh(k.stride()), *sbh(v.stride()), *sbh(o.stride()), int(window_size), _ptr(sink),
+        v.shape[3], _kernel_choice(kernel), 0, 0)
 
 
 # (Q/K head dim, V/O head dim) pairs the prefill kernels are built for:
@@ -463,7 +446,7 @@ def _attach_prefill_workspace(a, device, own=False):
 def _prefill(q, k, v, o, lse, scale, causal, layout, window_size=0, sink=None):
     a = _prefill_args(q, k, v, o, lse, scale, causal, layout, window_size, sink)
     _attach_prefill_workspace(a, q.device)
-    _lib.check(_lib.lib().fgqa_prefill_bf16(ctypes.byref(a), ctypes.c_void_p(_stream())), "fgqa_prefill_bf16")
+    _lib.check(_lib.lib().fgqa_prefill_bf16(ctypes.byref(a), _stream()), "fgqa_prefill_bf16")
 
 
 def _check_sink(sink, hq, dev):
@@ -518,7 +501,7 @@ def flash_gqa_forward_bshd(q, k, v, scale=None, out=None, lse=None, causal=True,
     per (device, stream), so calls on different streams may overlap."""
     a, out, lse, _keep = _prefill_bshd_prepare(q, k, v, scale, out, lse, causal, window_size, sink, kernel)
     _attach_prefill_workspace(a, q.device)
-    _lib.check(_lib.lib().fgqa_prefill_bf16(ctypes.byref(a), ctypes.c_void_p(_stream())), "fgqa_prefill_bf16")
+    _lib.check(_lib.lib().fgqa_prefill_bf16(ctypes.byref(a), _stream()), "fgqa_prefill_bf16")
     return out, lse
 
 
@@ -675,40 +658,19 @@ def _launch_bhsd_prefill(kind, q, k, v, scale, out, lse, causal):
 def _backward_args(q, k, v, o, lse, grad_o, dq, dk, dv, scale, causal, layout, workspace,
                    window_size=0, kv_head_split=0, dq_kernel="auto") -> _lib.BackwardArgs:
     """C ABI argument block; 4-D tensors in `layout` ('bshd' or 'bhsd')."""
-    def sbh(t):
-        if layout == "bshd":
-            return [t.stride(0), t.stride(1), t.stride(2)]
-        return [t.stride(0), t.stride(2), t.stride(1)]
-
     if layout == "bshd":
         B, Sq, Hq, D = q.shape
         _, Skv, Hkv, _ = k.shape
     else:
         B, Hq, Sq, D = q.shape
         _, Hkv, Skv, _ = k.shape
-    a = _lib.BackwardArgs()
-    a.q, a.k, a.v, a.o, a.lse, a.grad_o = (_ptr(x) for x in (q, k, v, o, lse, grad_o))
-    a.grad_q, a.grad_k, a.grad_v = _ptr(dq), _ptr(dk), _ptr(dv)
-    a.batch, a.seqlen_q, a.seqlen_kv = B, Sq, Skv
-    a.num_q_heads, a.num_kv_heads, a.head_dim = Hq, Hkv, D
-    a.causal = 1 if causal else 0
-    a.scale = float(scale)
-    a.window_size = int(window_size)
-    a.head_dim_v = int(v.shape[-1])
-    a.kv_head_split = int(kv_head_split)
-    a.dq_kernel = _kernel_choice(dq_kernel)
-    a.q_stride[:] = sbh(q)
-    a.k_stride[:] = sbh(k)
-    a.v_stride[:] = sbh(v)
-    a.o_stride[:] = sbh(o)
-    a.grad_o_stride[:] = sbh(grad_o)
-    a.grad_q_stride[:] = sbh(dq)
-    a.grad_k_stride[:] = sbh(dk)
-    a.grad_v_stride[:] = sbh(dv)
-    if workspace is not None:
-        a.workspace = workspace.data_ptr()
-        a.workspace_bytes = workspace.numel() * workspace.element_size()
-    return a
+    sbh = _SBH[layout]
+    return _lib.pack_backward(
+        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(grad_o), _ptr(dq), _ptr(dk), _ptr(dv),
+        B, Sq, Skv, Hq, Hkv, D, 1 if causal else 0, float(scale),
+        *sbh(q.stride()), *sbh(k.stride()), *sbh(v.stride()), *sbh(o.stride()), *sbh(grad_o.stride()),
+        *sbh(dq.stride()), *sbh(dk.stride()), *sbh(dv.stride()), *_workspace(workspace),
+        int(window_size), int(v.shape[-1]), int(kv_head_split), _kernel_choice(dq_kernel))
 
 
 def backward_workspace_bytes(batch, seqlen_q, seqlen_kv, num_q_heads, num_kv_heads, head_dim=128,
@@ -797,7 +759,7 @@ def flash_gqa_backward_bshd(q, k, v, o, lse, grad_o, scale=None, causal=True,
     a, grads, _keep = _backward_bshd_prepare(q, k, v, o, lse, grad_o, scale, causal,
                                              grad_q, grad_k, grad_v, workspace, window_size,
                                              kv_head_split, dq_kernel)
-    _lib.check(_lib.lib().fgqa_prefill_backward_bf16(ctypes.byref(a), ctypes.c_void_p(_stream())),
+    _lib.check(_lib.lib().fgqa_prefill_backward_bf16(ctypes.byref(a), _stream()),
                "fgqa_prefill_backward_bf16")
     return grads
 
@@ -877,7 +839,7 @@ def _launch_bhsd_backward(kind, q, k, v, o, lse, grad_o, scale, causal, window_s
     dv = torch.empty((batch, num_kv_heads, seqlen_kv, head_dim_v), device=qb.device, dtype=torch.bfloat16)
     a = _backward_args(qb, kb, vb, ob, lse_b, gb, dq, dk, dv, scale, causal, "bhsd", None,
                        int(window_size or 0))
-    _lib.check(_lib.lib().fgqa_prefill_backward_bf16(ctypes.byref(a), ctypes.c_void_p(_stream())),
+    _lib.check(_lib.lib().fgqa_prefill_backward_bf16(ctypes.byref(a), _stream()),
                "fgqa_prefill_backward_bf16")
     if squeeze_output:
         return dq.squeeze(0), dk.squeeze(0), dv.squeeze(0)
@@ -1036,30 +998,17 @@ def launch_flash_swa_forward_bf16_kernel(q, k, v, scale=None, out=None, lse=None
 # --------------------------------------------------------------------------- sparse-index prefill
 def _sparse_args(q, k, v, o, lse, idx, scale, causal, layout) -> _lib.SparsePrefillArgs:
     """C ABI argument block; q/k/v/o 4-D in `layout` ('bshd' or 'bhsd'), idx [B, Hkv, Sq, n]."""
-    def sbh(t):
-        if layout == "bshd":
-            return [t.stride(0), t.stride(1), t.stride(2)]
-        return [t.stride(0), t.stride(2), t.stride(1)]
-
     if layout == "bshd":
         B, Sq, Hq, D = q.shape
         _, Skv, Hkv, _ = k.shape
     else:
         B, Hq, Sq, D = q.shape
         _, Hkv, Skv, _ = k.shape
-    a = _lib.SparsePrefillArgs()
-    a.q, a.k, a.v, a.o, a.lse, a.kv_indices = (_ptr(x) for x in (q, k, v, o, lse, idx))
-    a.batch, a.seqlen_q, a.seqlen_kv = B, Sq, Skv
-    a.num_q_heads, a.num_kv_heads, a.head_dim = Hq, Hkv, D
-    a.num_sparse_kv = idx.shape[3]
-    a.causal = 1 if causal else 0
-    a.scale = float(scale)
-    a.q_stride[:] = sbh(q)
-    a.k_stride[:] = sbh(k)
-    a.v_stride[:] = sbh(v)
-    a.o_stride[:] = sbh(o)
-    a.idx_stride[:] = [idx.stride(0), idx.stride(1), idx.stride(2)]
-    return a
+    sbh = _SBH[layout]
+    return _lib.pack_sparse(
+        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(idx), B, Sq, Skv, Hq, Hkv, D, idx.shape[3],
+        1 if causal else 0, float(scale),
+        *sbh(q.stride()), *sbh(k.stride()), *sbh(v.stride()), *sbh(o.stride()), *idx.stride()[:3])
 
 
 def _check_indices(idx, B, Hkv, Sq):
@@ -1106,7 +1055,7 @@ def flash_sgqa_forward_bshd(q, k, v, kv_indices, scale=None, out=None, lse=None,
     int32 [B,Hkv,Sq,n] (key lists shared by a KV head's query heads; entries
     < 0, >= Skv or, if causal, > the row are skipped) -> (out [B,Sq,Hq,D], lse [B,Hq,Sq])."""
     a, out, lse, _keep = _sparse_bshd_prepare(q, k, v, kv_indices, scale, out, lse, causal)
-    _lib.check(_lib.lib().fgqa_sparse_prefill_bf16(ctypes.byref(a), ctypes.c_void_p(_stream())),
+    _lib.check(_lib.lib().fgqa_sparse_prefill_bf16(ctypes.byref(a), _stream()),
                "fgqa_sparse_prefill_bf16")
     return out, lse
 
@@ -1219,7 +1168,7 @@ def launch_flash_sgqa_forward_bf16_kernel(q, k, v, sparse_kv_indices, num_sparse
         qb, kb, vb = _prep(qb), _prep(kb), _prep(vb)
         idx = sparse_kv_indices if sparse_kv_indices.stride(3) == 1 else sparse_kv_indices.contiguous()
         a = _sparse_args(qb, kb, vb, out_b, lse_b, idx, scale, causal, "bhsd")
-        _lib.check(_lib.lib().fgqa_sparse_prefill_bf16(ctypes.byref(a), ctypes.c_void_p(_stream())),
+        _lib.check(_lib.lib().fgqa_sparse_prefill_bf16(ctypes.byref(a), _stream()),
                    "fgqa_sparse_prefill_bf16")
     if squeeze_output:
         return out_b.squeeze(0), lse_b.squeeze(0)
