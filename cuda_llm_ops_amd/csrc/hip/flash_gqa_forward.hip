@@ -1339,7 +1339,7 @@ extern "C" int fgqa_prefill_kernel_choice(const fgqa_prefill_args* a, int32_t* k
     if (kernel == nullptr) return FGQA_ERR_INVALID_ARGUMENT;
     const int cus = device_cu_count();
     if (cus <= 0) return FGQA_ERR_HIP;
-    const fgqa_prefill_args pa = plan::prefill_padded(a) ? plan::padded_args(a) : *a;
+    const fgqa_prefill_args pa = plan::prefill_padded(a) && !plan::prefill_native64(a) ? plan::padded_args(a) : *a;
     *kernel = plan::prefill_choice(&pa, cus);
     return FGQA_OK;
 }
@@ -1350,7 +1350,7 @@ extern "C" int fgqa_prefill_kernel_name(const fgqa_prefill_args* a, const char**
     if (name == nullptr) return FGQA_ERR_INVALID_ARGUMENT;
     const int cus = device_cu_count();
     if (cus <= 0) return FGQA_ERR_HIP;
-    const fgqa_prefill_args pa = plan::prefill_padded(a) ? plan::padded_args(a) : *a;
+    const fgqa_prefill_args pa = plan::prefill_padded(a) && !plan::prefill_native64(a) ? plan::padded_args(a) : *a;
     *name = plan::prefill_kernel_name(&pa, cus);
     return FGQA_OK;
 }

@@ -339,12 +339,14 @@ int validate_prefill(const fgqa_prefill_args* a) {
     return FGQA_OK;
 }
 
-int64_t wide_pairs(const fgqa_prefill_args* a) {
+// Units of 256 rows (up to 8 heads of a KV head side by side).
+static int64_t wide_units(const fgqa_prefill_args* a) {
     const int group = a->num_q_heads / a->num_kv_heads;
     const int hbw = group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-    const int64_t units = ceil_div(a->seqlen_q, 256 / hbw) * (int64_t)(group / hbw) * a->num_kv_heads * a->batch;
-    return (units + 1) / 2;
+    return ceil_div(a->seqlen_q, 256 / hbw) * (int64_t)(group / hbw) * a->num_kv_heads * a->batch;
 }
+
+int64_t wide_pairs(const fgqa_prefill_args* a) { return (wide_units(a) + 1) / 2; }
 
 bool wide_on_pairs(const fgqa_prefill_args* a, int cus) {
     const int64_t pairs = wide_pairs(a);
@@ -353,7 +355,75 @@ bool wide_on_pairs(const fgqa_prefill_args* a, int cus) {
 
 bool tall_on_pairs(const fgqa_prefill_args* a, int cus) { return a->causal && wide_on_pairs(a, cus); }
 
-// The caller's `kernel`, or for AUTO the choice by grid size:
+// AUTO for the kernels built for head dim 64 without a window or sink, by the
+// 128-row units and the query rows S (a unit's steps).  Two units share a CU in
+// the whole-range kernel there (half the LDS and registers of head dim 128's),
+// so it wins as soon as the grid gives every CU more than one unit, where the
+// split kernel needs a second round.  Measured on 430 grids (Hq/Hkv 16/1, 32/8,
+// 16/16 and 8/8, B 1-4, S 64-8192, 256 CUs; us, whole / split / wide):
+//  - up to 448 keys (7 tiles): whole; the split kernel's two groups have too
+//    little to share for their merge.  S = 128, 32 units 5.9 / 7.4 / 9.5;
+//    S = 400, 104 units 9.2 / 9.7 / 14.8; at 512 10.4 / 10.0 / 15.5: split.
+//  - a unit per CU or fewer: split.  S = 2048, 256 units 29 / 23 / 28.
+//  - causal, just above: the diagonal leaves the split kernel's second units
+//    room, the more the longer the sequence.  S = 777, 400 units 15.7 / 17.5 /
+//    19.2, but S = 1536, 384 units 24 / 20.5 / 24.
+//  - 2 units per CU over long sequences, causal up to 4 at 4096 rows: the
+//    256-row kernel balances its units' lengths.  S = 4096 causal, 512 units
+//    60 / 49 / 50, 1024 units 85 / 95 / 82; S = 4096 full, 512 units 86 / 91 / 79.
+//  - the rest: whole.  S = 1280 causal, 1280 units 38 / 57 / 49.
+static int choice_native64(const fgqa_prefill_args* a, int64_t units, int64_t cus) {
+    const int64_t s = a->seqlen_q;
+    if (a->seqlen_kv <= 448) return FGQA_KERNEL_WHOLE;
+    if (!a->causal) {
+        if (units <= cus) return FGQA_KERNEL_SPLIT;
+        return s >= 1536 && units <= 2 * cus ? FGQA_KERNEL_WIDE : FGQA_KERNEL_WHOLE;
+    }
+    if (units <= cus || (s >= 1024 && 2 * units <= 3 * cus) || (s >= 1536 && units < 2 * cus))
+        return FGQA_KERNEL_SPLIT;
+    if ((s >= 1536 && units <= 2 * cus) || (s >= 4096 && units <= 4 * cus)) return FGQA_KERNEL_WIDE;
+    return FGQA_KERNEL_WHOLE;
+}
+
+// AUTO's short sequences and full (non-causal) grids at head dim 128 without a
+// window or sink; AUTO: none of them, the general lines of prefill_choice.
+// Measured on 780 grids (as above, also Hq/Hkv 28/4 and 16/2, B up to 8; us,
+// whole / split / wide):
+//  - a unit per CU or fewer: the split kernel halves a unit's steps but pays
+//    for the merge; up to 5 tiles of 64 keys, or 7 (4 + 3), there is nothing to
+//    gain.  S = 192, 128 units 8.4 / 10.0 / 13.2; S = 300, 80 units 10.4 / 11.4 /
+//    14.4; S = 448 12.3 / 13.1 / 18.4; but 6 tiles 11.6 / 11.3 / 17.5.
+//  - causal, above that and up to two per CU: two units share a CU, one in the
+//    shadow of the other, while the split kernel runs them in turn, and the
+//    wide kernel's longest unit is the whole launch.  S = 300, 320 units 12.7 /
+//    16.1 / 16.3; S = 777, 400 units 21.6 / 23.0 / 23.8.  From 10 tiles the
+//    split kernel keeps grids that its second round does not fill (S = 640, 320
+//    units 18.4 / 17.9 / 21.5); at 1024 rows, 512 units 28.0 / 28.8 / 27.7.
+//  - causal, more units: the wide kernel, unless its taller units add padding
+//    (S = 777 with one head to a unit, 784 units: 37.6 / 45.9 / 42.8).
+//  - full: whole up to 6 tiles (S = 300, 384 units 16.1 / 24.7 / 19.2), else
+//    wide (S = 1536, 384 units 47 / 48 / 42; S = 2048, 1024 units 134 / 134 / 121),
+//    unless its last round is mostly empty (S = 1280, 640 units 65 / 66 / 67) or
+//    its units mostly padding.  Then the split kernel only for long sequences
+//    (S = 6000, 752 units 272 / 259 / 270; S = 520, 544 units 33 / 43 / 37).
+//    Grids of more than 32 units per CU keep the whole-range kernel, which
+//    fgqa_prefill_kernel_choice has always reported for them (64 per CU: 16.0
+//    ms against 14.1).
+static int choice_short_or_full(const fgqa_prefill_args* a, int64_t units, int64_t cus) {
+    const int64_t s = a->seqlen_q, tiles = ceil_div(a->seqlen_kv, 64), wu = wide_units(a);
+    if (units <= cus) return tiles <= 5 || tiles == 7 ? FGQA_KERNEL_WHOLE : FGQA_KERNEL_AUTO;
+    if (a->causal) {
+        if (units > 2 * cus) return 200 * wu > 108 * units ? FGQA_KERNEL_WHOLE : FGQA_KERNEL_AUTO;
+        return s <= 576 || (s <= 960 && 2 * units >= 3 * cus) ? FGQA_KERNEL_WHOLE : FGQA_KERNEL_AUTO;
+    }
+    if (tiles <= 6) return FGQA_KERNEL_WHOLE;
+    if (units > 32 * cus) return FGQA_KERNEL_AUTO;
+    if (8 * wu <= 5 * units && (wu <= cus || 20 * wu >= 17 * cus * ceil_div(wu, cus))) return FGQA_KERNEL_WIDE;
+    return s <= 1024 ? FGQA_KERNEL_WHOLE : FGQA_KERNEL_AUTO;
+}
+
+// The caller's `kernel`, or for AUTO the choice by grid size: choice_native64
+// and choice_short_or_full above for what they cover, else
 //  - wide: causal, no window or sink, and the wide kernel's unit pairs fill
 //    the CUs (two workgroups per pair, within 1/8 of one per CU).  Forced, it
 //    also runs the window / sink form;
@@ -374,6 +444,9 @@ int prefill_choice(const fgqa_prefill_args* a, int cus) {
     const bool win = a->window_size > 0;
     const bool swa = win || a->sink != nullptr;
     const int64_t units = ceil_div(a->seqlen_q, 128 / hb) * (int64_t)(group / hb) * a->num_kv_heads * a->batch;
+    if (!swa && prefill_native64(a)) return choice_native64(a, units, cus);
+    if (!swa && a->head_dim == kHeadDim)
+        if (const int k = choice_short_or_full(a, units, cus); k != FGQA_KERNEL_AUTO) return k;
     const int64_t pairs = wide_pairs(a);
     const int64_t wide_grid = 16 * ceil_div(pairs, 8);
     if (!swa && a->causal && pairs <= kPrefillMaxSplit && wide_grid <= cus && 8 * wide_grid >= 7 * (int64_t)cus)

@@ -42,9 +42,12 @@ enum fgqa_status {
  * `dq_kernel`).  AUTO picks by grid size; the others force one kernel shape,
  * for tuning and tests.  Callers that zero the argument struct get AUTO.
  *   FGQA_KERNEL_WHOLE  one workgroup runs a 128-row unit over its whole KV range
+ *                      (AUTO's choice for short sequences, with a window, and
+ *                      at head dims up to 64 for most grids of more than a
+ *                      unit per CU)
  *   FGQA_KERNEL_SPLIT  two wave groups run the two halves of a unit's KV range
- *                      and merge (the choice for causal grids under 2 units
- *                      per CU and non-causal grids under 4)
+ *                      and merge (AUTO's choice for longer sequences with up
+ *                      to one unit per CU, causal ones up to two)
  *   FGQA_KERNEL_WIDE   (prefill forward) two wave groups
  *                      share each K/V tile of a 256-row unit.  With at most
  *                      one unit pair per two CUs (and at most 128 pairs) a
@@ -52,8 +55,9 @@ enum fgqa_status {
  *                      merge through device memory the library holds (calls
  *                      that overlap on one device must not both use it);
  *                      larger grids run whole units on a persistent grid
- *                      (AUTO's choice for causal grids without a window or
- *                      sink from 2 units per CU)
+ *                      (AUTO's choice without a window or sink for most
+ *                      causal grids from 2 units per CU, and non-causal
+ *                      ones from 1, at head dim 128)
  *   FGQA_KERNEL_TALL   (prefill forward, head_dim 128, no window or sink) the
  *                      256-row units of FGQA_KERNEL_WIDE on four waves of 64
  *                      rows each, one wave per SIMD, each K/V operand read

@@ -371,6 +371,59 @@ static void test_prefill_known_shapes() {
     CHECK(plan::prefill_choice(&ws, kCus) == FGQA_KERNEL_WHOLE);
 }
 
+// AUTO's lines for head dim 64 and for full grids at 128, a step on either
+// side of each; over many grids, the merge scratch that head dim 64's choice
+// needs is within what the copies' layout holds.
+static void test_prefill_choice_lines() {
+    auto args64 = [](int B, int S, int hq, int hkv, bool causal) {
+        fgqa_prefill_args a = prefill_args(B, S, hq, hkv, causal);
+        a.head_dim = a.head_dim_v = 64;
+        return a;
+    };
+    struct Line { int B, S, hq, hkv; bool causal; int want; };
+    const Line at64[] = {
+        {1, 448, 16, 1, true, FGQA_KERNEL_WHOLE},   {1, 449, 16, 1, true, FGQA_KERNEL_SPLIT},
+        {1, 2048, 16, 1, true, FGQA_KERNEL_SPLIT},  {2, 640, 32, 8, true, FGQA_KERNEL_WHOLE},
+        {1, 1536, 32, 8, true, FGQA_KERNEL_SPLIT},  {2, 1535, 32, 8, true, FGQA_KERNEL_WHOLE},
+        {1, 2048, 32, 8, true, FGQA_KERNEL_WIDE},   {1, 2080, 32, 8, true, FGQA_KERNEL_WHOLE},
+        {1, 4096, 32, 8, true, FGQA_KERNEL_WIDE},   {1, 4128, 32, 8, true, FGQA_KERNEL_WHOLE},
+        {1, 1024, 32, 8, false, FGQA_KERNEL_SPLIT}, {1, 1025, 32, 8, false, FGQA_KERNEL_WHOLE},
+        {1, 1536, 32, 8, false, FGQA_KERNEL_WIDE},  {1, 2080, 32, 8, false, FGQA_KERNEL_WHOLE},
+    };
+    for (const Line& l : at64) {
+        const fgqa_prefill_args a = args64(l.B, l.S, l.hq, l.hkv, l.causal);
+        CHECK(plan::validate_prefill(&a) == FGQA_OK);
+        CHECK(plan::prefill_choice(&a, kCus) == l.want);
+    }
+    const Line at128[] = {
+        {1, 320, 32, 8, true, FGQA_KERNEL_WHOLE},   {1, 321, 32, 8, true, FGQA_KERNEL_SPLIT},
+        {1, 448, 32, 8, false, FGQA_KERNEL_WHOLE},  {1, 449, 32, 8, false, FGQA_KERNEL_SPLIT},
+        {2, 576, 32, 8, true, FGQA_KERNEL_WHOLE},   {2, 577, 32, 8, true, FGQA_KERNEL_SPLIT},
+        {2, 737, 32, 8, true, FGQA_KERNEL_WHOLE},   {2, 736, 32, 8, true, FGQA_KERNEL_SPLIT},
+        {2, 960, 32, 8, true, FGQA_KERNEL_WHOLE},   {2, 961, 32, 8, true, FGQA_KERNEL_WIDE},
+        {4, 777, 28, 4, true, FGQA_KERNEL_WHOLE},   {4, 1024, 28, 4, true, FGQA_KERNEL_WIDE},
+        {4, 384, 32, 8, false, FGQA_KERNEL_WHOLE},  {4, 448, 32, 8, false, FGQA_KERNEL_WIDE},
+        {4, 520, 32, 8, false, FGQA_KERNEL_WHOLE},
+        {1, 1024, 32, 8, false, FGQA_KERNEL_SPLIT}, {1, 1025, 32, 8, false, FGQA_KERNEL_WIDE},
+        {1, 2048, 32, 8, false, FGQA_KERNEL_WIDE},  {1, 2080, 32, 8, false, FGQA_KERNEL_SPLIT},   // 1.02 rounds
+        {4, 8192, 32, 8, false, FGQA_KERNEL_WIDE},  {4, 8224, 32, 8, false, FGQA_KERNEL_WHOLE},
+        {32, 300, 16, 16, false, FGQA_KERNEL_WHOLE},   // units of one head: 2 x 256 rows for 3 x 128
+    };
+    for (const Line& l : at128) {
+        const fgqa_prefill_args a = prefill_args(l.B, l.S, l.hq, l.hkv, l.causal);
+        CHECK(plan::prefill_choice(&a, kCus) == l.want);
+    }
+    for (const int hq : {16, 8, 6, 3})
+        for (const int hkv : {1, 2, 8})
+            for (int S = 1; S < 9000; S += 1 + S / 5)
+                for (const bool causal : {true, false}) {
+                    const fgqa_prefill_args a = args64(2, S, hq * hkv, hkv, causal);
+                    const fgqa_prefill_args c = plan::padded_args(&a);
+                    CHECK(plan::merge_scratch_bytes(&a, plan::prefill_choice(&a, kCus), kCus) <=
+                          plan::merge_scratch_bytes(&c, plan::prefill_choice(&c, kCus), kCus));
+                }
+}
+
 static void test_prefill_rejections() {
     const fgqa_prefill_args a = prefill_args(1, 4096, 16, 1, true);
     fgqa_prefill_args b = a;
@@ -907,6 +960,7 @@ int main() {
     test_decode_extremes();
     test_paged();
     test_prefill_known_shapes();
+    test_prefill_choice_lines();
     test_prefill_rejections();
     test_prefill_padded_head_dims();
     test_backward();

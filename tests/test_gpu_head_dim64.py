@@ -18,7 +18,9 @@ def _both(cuda, B, Sq, Skv, Hq, Hkv, dqk, dv, **kw):
                for s in ((B, Sq, Hq, dqk), (B, Skv, Hkv, dqk), (B, Skv, Hkv, dv)))
     out, lse = fg.flash_gqa_forward_bshd(q, k, v, **kw)
     wide = torch.full((B, Sq, Hq, dv + 3), 7.0, device=cuda, dtype=torch.bfloat16)
-    out2, lse2 = fg.flash_gqa_forward_bshd(q, k, v, out=wide[..., :dv], **kw)
+    # (AUTO may choose another kernel shape for the copies)
+    kw2 = dict(kw, kernel=fg.prefill_kernel_choice(q, k, v, **kw))
+    out2, lse2 = fg.flash_gqa_forward_bshd(q, k, v, out=wide[..., :dv], **kw2)
     torch.cuda.synchronize()
     assert torch.isfinite(out.float()).all()
     assert torch.equal(out.view(torch.int16), out2.contiguous().view(torch.int16))
