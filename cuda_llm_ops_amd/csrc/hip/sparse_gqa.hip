@@ -12,18 +12,25 @@
 // One wave owns one work item: a query position, a KV head and up to 16 of
 // its query heads, which share the position's index list.  The heads are the
 // N dimension of v_mfma_f32_16x16x32_bf16; per 32-entry step:
-//   S^T (32 keys x 16 heads) = K_gathered . Q^T     8 MFMAs, K from the wave's
-//                                                    LDS tile (b128 reads)
+//   S^T (32 keys x 16 heads) = K_gathered . Q^T     8 MFMAs, K transposed within
+//                                                    lane quads in registers
 //   O^T (128 x 16)          += V^T . P^T            8 MFMAs, V read transposed
-//                                                    from its LDS tile
+//                                                    from the wave's LDS tile
 //                                                    (ds_read_b64_tr_b16)
-// The next step's K and V rows are in flight while a step is computed.  Each
-// step reads 16 KB of K/V rows; the MFMA work per step is small, so the kernel
-// is bound by how fast the gathers are served (mostly from L2 and the MALL:
-// every position gathers rows of the same Skv x 256-byte K/V).
-#include <limits.h>
+// The next step's K and V rows are in flight while a step is computed.
+//
+// What bounds it: each step gathers 16 KB of K/V rows and does little with
+// them.  At S = 16384, 512 entries (4.3 GB of gathers) the gathers alone take
+// 129 us when they all hit L1, the steps without gathers 112 us; together 155 us
+// from L1 and 189 us from the real lists (L2 misses; 4 MB of L2 per XCD against
+// 8 MB of K/V).  Before, K went through LDS as well (32 KB of LDS traffic per
+// step was the bound: 150 us without any gather) at two waves per SIMD, and
+// every list was sorted (37 us): 224 us.  Three waves per SIMD: 165 VGPRs, 11.3
+// KB of LDS.
 #include <math.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "fgqa_device.h"
 #include "fgqa_internal.h"
@@ -44,32 +51,47 @@ struct SparseParams {
     int64_t i_sb, i_sh, i_ss;   // index list strides: batch, kv head, query row
     int batch, sq, skv, hq, hkv, group, nsparse, causal;
     int n_hg;                   // ceil(group / 16) head groups per position
-    int n_steps;                // ceil(nsparse / 32), rounded up to even
     int64_t n_items;            // batch * hkv * sq * n_hg
+    int n_windows, window_shift;   // key windows a list is ordered by, 2^window_shift keys each
+    FastDiv div_hg, div_sq, div_hkv;
     float scale_log2;           // |scale| * log2(e)
     uint32_t q_sign;            // 0x80008000 when scale < 0 (Q is negated on load)
 };
 
 constexpr int kSpWaves = 4;                  // waves (= work items) per workgroup
 constexpr int kSpStep = 32;                  // index entries per step
-constexpr int kSpKRow = 288;                 // K row stride in LDS (256 + 32 bytes)
-constexpr int kSpVRow = 288;                 // V row stride in LDS
-constexpr int kSpKBytes = kSpStep * kSpKRow;
-constexpr int kSpVBytes = kSpStep * kSpVRow;
-constexpr int kSpIdxBytes = kSpStep * 4;
-constexpr int kSpWaveBytes = kSpKBytes + kSpVBytes + kSpIdxBytes;   // 17.9 KB of LDS per wave
-constexpr float kSpRescaleSlack = 8.f;       // log2 units: P <= 2^8 between rescales
+constexpr int kSpRow = 288;                  // K / V row stride in LDS (256 + 32 bytes)
+constexpr int kSpTileBytes = kSpStep * kSpRow;
+constexpr int kSpList = 512;                 // index entries taken (and ordered) at a time
+constexpr int kSpWaveBytes = kSpTileBytes + kSpList * 4 + 16;   // 11.3 KB of LDS per wave (and a word to drop entries in)
+constexpr float kSpMaxP = 65536.f;           // a lane's P of one step, before the max moves
 
-// Gathers are row-contiguous: load instruction i of a step fetches entries
-// 4i .. 4i+3, 16 lanes per 256-byte row, so every 16 lanes read two whole
-// 128-byte lines (a lane-per-row gather makes the L1 handle one access per
-// lane and is several times slower).  The rows then go through the wave's LDS
-// tiles to reach the MFMA operand layouts.  A 288-byte row stride (256 + 32)
-// keeps every LDS pattern here free of bank conflicts (SQ_LDS_BANK_CONFLICT
-// reads 0 for the b128 writes of one row's 16 chunks, the b128 A-operand reads
-// of 16 rows at one chunk, and the transposed reads of rows 0..7 x chunks
-// {2dt, 2dt + 1} per 32 lanes; a 272-byte stride costs the b128 reads 4
-// conflict cycles each).
+// Lists are taken window by window of keys where K/V outgrow an XCD's L2: all
+// waves of the XCD then walk the keys of their prefixes from low to high at
+// about the same pace, and a row one wave fetches is often still in L2 when
+// another needs it.  Windows of 2048 keys (1 MB of K/V; S = 16384, 512 entries:
+// 189 us against 194 with 4096 keys, 193 with 1024, 221 without windows, 202
+// fully sorted), but none for fewer than 32 of a list's entries (a window costs
+// ~60 instructions: S = 24576, 64 entries 104 us with 12 windows, 90 with 2).
+// Up to 8192 keys all K/V fit: one window.
+constexpr int kSpWindowLog2 = 11;
+constexpr int kSpNoWindows = 8192;
+// Two waves per SIMD instead of three (kPerSimd below): a wave's next K rows are
+// gathered before its scores instead of after them (188 registers).  Chosen
+//  - for grids that fit the chip at two workgroups per CU, where a launch is one
+//    wave's chain of steps: S = 546, 512 entries 19.2 against 21.3 us, S = 2048,
+//    512 entries 29.2 against 31.1; at S = 3000 (750 workgroups) 15.3 against 14.6;
+//  - past 32768 keys, where L2 serves fewer waves better: 65536 keys, 512 entries
+//    1202 against 1371 us (the former kernel, sorted lists and two steps in
+//    flight: 1182), 1024 entries 2582 against 2729; 16384 keys: 199 against 188.
+constexpr int kSpManyKeys = 32768;
+
+// Gathers read whole rows per instruction, in pieces of a quad (K, 64 bytes) or
+// of 16 lanes (V, 256 bytes); both run at the same rate (129-132 us for 4.3 GB
+// from L1), while a lane-per-row gather makes the L1 handle one access per lane
+// and is several times slower.  A 288-byte row stride (256 + 32) keeps both LDS
+// patterns of V free of bank conflicts (the b128 writes of one row's 16 chunks,
+// and the transposed reads of rows 0..7 x chunks {2dt, 2dt + 1} per 32 lanes).
 
 // Block -> first work item: the last positions first.  Blocks go round-robin
 // over the 8 XCDs, so every XCD works through the same positions at the same
@@ -83,92 +105,96 @@ __device__ __forceinline__ int64_t sp_block_first_item(int64_t nblocks) {
     return (nblocks - 1 - (int64_t)blockIdx.x) * kSpWaves;
 }
 
-// The value of lane ^ d: DPP quad permutes for d = 1, 2, a bit-mode swizzle
-// inside each half-wave for 4 <= d <= 16, the half-wave swap for 32.
-__device__ __forceinline__ int sp_xor(int v, int d, int lane) {
-    switch (d) {
-        case 1: return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
-        case 2: return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
-        case 4: return __builtin_amdgcn_ds_swizzle(v, (4 << 10) | 0x1F);
-        case 8: return __builtin_amdgcn_ds_swizzle(v, (8 << 10) | 0x1F);
-        case 16: return __builtin_amdgcn_ds_swizzle(v, (16 << 10) | 0x1F);
-        default: {
-            const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
-            return (int)(lane < 32 ? r[1] : r[0]);
-        }
-    }
+// Lanes 4a .. 4a+3 hold, in r[i], dword c of chunk j of row i (lane 4a + j);
+// afterwards lane 4a + j holds chunk i of row j in r[i].  Two dwords (a and b) at
+// a time: each of the 16 moves takes the neighbour's register through DPP and
+// keeps or replaces by a lane mask (v_cndmask with a DPP source; the masks go
+// through vcc).  A DPP read needs two wait states after a VALU write of its
+// register: the s_nop covers what comes before, the order of the moves the rest.
+__device__ __forceinline__ void sp_transpose_quad(uint32_t& a0, uint32_t& a1, uint32_t& a2, uint32_t& a3,
+                                                  uint32_t& b0, uint32_t& b1, uint32_t& b2, uint32_t& b3,
+                                                  uint64_t bit0, uint64_t bit1) {
+    uint32_t t0, t1, t2, t3, u0, u1, u2, u3;
+    asm("s_not_b64 vcc, %[m0]\n\t"
+        "s_nop 1\n\t"
+        "v_cndmask_b32_dpp %[t0], %[a1], %[a0], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[t2], %[a3], %[a2], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[u0], %[b1], %[b0], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[u2], %[b3], %[b2], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_mov_b64 vcc, %[m0]\n\t"
+        "v_cndmask_b32_dpp %[t1], %[a0], %[a1], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[t3], %[a2], %[a3], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[u1], %[b0], %[b1], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[u3], %[b2], %[b3], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_not_b64 vcc, %[m1]\n\t"
+        "v_cndmask_b32_dpp %[a0], %[t2], %[t0], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[a1], %[t3], %[t1], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b0], %[u2], %[u0], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b1], %[u3], %[u1], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_mov_b64 vcc, %[m1]\n\t"
+        "v_cndmask_b32_dpp %[a2], %[t0], %[t2], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[a3], %[t1], %[t3], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b2], %[u0], %[u2], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b3], %[u1], %[u3], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+        : [a0] "+v"(a0), [a1] "+v"(a1), [a2] "+v"(a2), [a3] "+v"(a3), [b0] "+v"(b0), [b1] "+v"(b1), [b2] "+v"(b2),
+          [b3] "+v"(b3), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3), [u0] "=&v"(u0),
+          [u1] "=&v"(u1), [u2] "=&v"(u2), [u3] "=&v"(u3)
+        : [m0] "s"(bit0), [m1] "s"(bit1)
+        : "vcc", "scc");
 }
 
-// Ascending bitonic sort of a wave's 512 ints, value 8*lane + r in x[r]:
-// distances of 8 values or more pair registers across lanes, smaller ones
-// pair registers of a lane.  Deterministic (no atomics).
-__device__ __forceinline__ void sp_sort512(int (&x)[8], int lane) {
-#pragma unroll
-    for (int k = 2; k <= 512; k <<= 1)
-#pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            if (j >= 8) {
-                // value e pairs with e ^ j: same register of lane ^ (j / 8);
-                // the block of size k holding e sorts up when (e & k) == 0
-                const int d = j >> 3;
-                const bool keep_min = ((lane & d) == 0) == ((lane & (k >> 3)) == 0);
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const int o = sp_xor(x[r], d, lane);
-                    x[r] = keep_min ? min(x[r], o) : max(x[r], o);
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    if (r & j) continue;
-                    const bool up = ((8 * lane + r) & k) == 0;
-                    const int lo = min(x[r], x[r | j]), hi = max(x[r], x[r | j]);
-                    x[r] = up ? lo : hi;
-                    x[r | j] = up ? hi : lo;
-                }
-            }
-        }
-}
-
-// kSorted: lists of at most 512 entries, taken in ascending key order (see
-// the loop below); otherwise in list order, streamed a step ahead.
-template <bool kSorted>
-__global__ __launch_bounds__(kSpWaves * kWave, 2) void sparse_prefill_kernel(SparseParams p) {
+// kSameRows: K and V rows are the same number of bytes apart, so one offset
+// (kept in the list instead of the key) addresses both.  kPerSimd: waves per
+// SIMD, see kSpManyKeys.
+template <bool kSameRows, int kPerSimd>
+__global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_kernel(SparseParams p) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[kSpWaves * kSpWaveBytes];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int64_t item = sp_block_first_item(gridDim.x) + wave;
     if (item >= p.n_items) return;   // the kernel has no barrier: a finished wave may leave
-    unsigned char* kl = smem + wave * kSpWaveBytes;
-    unsigned char* vl = kl + kSpKBytes;
-    int* il = reinterpret_cast<int*>(vl + kSpVBytes);
+    unsigned char* tile = smem + wave * kSpWaveBytes;   // a step's V rows
+    int* il = reinterpret_cast<int*>(tile + kSpTileBytes);
 
     // (the divisions run on the VALU: readfirstlane tells the compiler the
     // results are wave-uniform, so buffer descriptors stay in SGPRs)
-    int64_t rest = item;
-    const int hg = __builtin_amdgcn_readfirstlane((int)(rest % p.n_hg));
-    rest /= p.n_hg;
-    const int pos = __builtin_amdgcn_readfirstlane((int)(rest % p.sq));
-    rest /= p.sq;
-    const int kvh = __builtin_amdgcn_readfirstlane((int)(rest % p.hkv));
-    const int b = __builtin_amdgcn_readfirstlane((int)(rest / p.hkv));
+    int hg, pos, kvh, b;
+    if (p.n_items < ((int64_t)1 << 31)) {
+        const int r0 = fast_div((int)item, p.div_hg), r1 = fast_div(r0, p.div_sq), r2 = fast_div(r1, p.div_hkv);
+        hg = (int)item - r0 * p.n_hg;
+        pos = r0 - r1 * p.sq;
+        kvh = r1 - r2 * p.hkv;
+        b = r2;
+    } else {
+        int64_t rest = item;
+        hg = (int)(rest % p.n_hg);
+        rest /= p.n_hg;
+        pos = (int)(rest % p.sq);
+        rest /= p.sq;
+        kvh = (int)(rest % p.hkv);
+        b = (int)(rest / p.hkv);
+    }
+    hg = __builtin_amdgcn_readfirstlane(hg);
+    pos = __builtin_amdgcn_readfirstlane(pos);
+    kvh = __builtin_amdgcn_readfirstlane(kvh);
+    b = __builtin_amdgcn_readfirstlane(b);
 
     const int l16 = lane & 15;
     const int g = lane >> 4;          // 16-lane group
-    const int l32 = lane & 31;
     const int h0 = kvh * p.group + hg * 16;
     const int nh = min(16, p.group - hg * 16);   // real heads in this item
 
-    // Q^T as the B operand: lane (head l16, group g) holds dims 32*ks + 8g .. +7.
+    // Q^T as the B operand: lane (head l16, group g) holds dims 32g + 8ks .. +7
+    // of k-step ks, as the K operand below.
     bf16x8_t qop[4];
     {
         const __amdgpu_buffer_rsrc_t qrs =
             make_rsrc(p.q + b * p.q_sb + (int64_t)pos * p.q_ss + (int64_t)h0 * p.q_sh,
                       (uint32_t)((int64_t)(nh - 1) * p.q_sh * 2 + 256));
-        const uint32_t qoff = (uint32_t)((int64_t)min(l16, nh - 1) * p.q_sh * 2) + g * 16;
+        const uint32_t qoff = (uint32_t)((int64_t)min(l16, nh - 1) * p.q_sh * 2) + g * 64;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            u32x4_t t = buf_load16(qrs, qoff + ks * 64);
+            u32x4_t t = buf_load16(qrs, qoff + ks * 16);
             t = (l16 < nh) ? (t ^ p.q_sign) : u32x4_t{0u, 0u, 0u, 0u};
             qop[ks] = as_bf16x8(t);
         }
@@ -188,53 +214,47 @@ __global__ __launch_bounds__(kSpWaves * kWave, 2) void sparse_prefill_kernel(Spa
     const __amdgpu_buffer_rsrc_t krs = make_rsrc(p.k + b * p.k_sb + kvh * p.k_sh, k_bytes);
     const __amdgpu_buffer_rsrc_t vrs = make_rsrc(p.v + b * p.v_sb + kvh * p.v_sh, v_bytes);
 
-    // Index lists of steps t and t + 1 (t even): lane l loads entry 32t + l.
-    auto load_pair = [&](int t) -> int {
-        return (int)__builtin_amdgcn_raw_buffer_load_b32(irs, (uint32_t)(t * kSpStep + lane) * 4, 0, 0);
+    // Row gathers of step t.  K: instruction (tt, i), lane 4a + j of group g
+    // reads chunk 4g + j of entry 16tt + 4a + i (a quad reads 64 bytes of one
+    // row, the wave four whole rows); the quad's transposition then leaves entry
+    // 16tt + l16 in lane l16, the MFMA's A operand with dims 32g + 8ks .. +7 in
+    // register ks.  V: instruction i, group g reads entry 8g + i, a row per 16
+    // lanes, into the same row of the LDS tile.
+    u32x4_t kr[2][4], vr[8];
+    auto issue_k = [&](int t) {
+        const u32x4_t* w = reinterpret_cast<const u32x4_t*>(il + t * kSpStep + (l16 & 12));
+        const u32x4_t r0 = w[0], r1 = w[4];
+        const uint32_t chunk = (uint32_t)(g * 64 + (lane & 3) * 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            kr[0][i] = buf_load16(krs, (kSameRows ? r0[i] : r0[i] * kss) + chunk);
+            kr[1][i] = buf_load16(krs, (kSameRows ? r1[i] : r1[i] * kss) + chunk);
+        }
     };
-    // Usable-entry masks of the pair: bit e of the low (high) word = entry
-    // 32t + e (32t + 32 + e).  Usable -> its key row, else row 0 (read, then masked).
-    auto pair_mask = [&](int t, int j) -> uint64_t {
-        const bool ok = (t * kSpStep + lane < p.nsparse) && j >= 0 && j < p.skv && (!p.causal || j <= pos);
-        return __builtin_amdgcn_ballot_w64(ok);
-    };
-    // Leaves the key rows of step t (half = 0) or t + 1 (half = 1) in the index
-    // area, stored so that lane l finds the rows of entries 4i + l/16 (i = 0..7)
-    // in 8 consecutive words.
-    auto post_rows = [&](int j, uint64_t mask, int half) {
-        if ((lane >> 5) == half) il[(l32 & 3) * 8 + (l32 >> 2)] = ((mask >> lane) & 1u) ? j : 0;
-    };
-
-    // Row gathers of one step: instruction i, lane l -> entry 4i + l/16,
-    // 16-byte chunk l % 16, into one of two register sets (two steps in flight).
-    struct Rows {
-        u32x4_t k[8], v[8];
-    };
-    Rows ra, rb;
-    auto issue = [&](Rows& r) {
-        const u32x4_t r0 = *reinterpret_cast<const u32x4_t*>(il + (lane >> 4) * 8);
-        const u32x4_t r1 = *reinterpret_cast<const u32x4_t*>(il + (lane >> 4) * 8 + 4);
+    auto issue_v = [&](int t) {
+        const u32x4_t* w = reinterpret_cast<const u32x4_t*>(il + t * kSpStep + g * 8);
+        const u32x4_t r0 = w[0], r1 = w[1];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const uint32_t row = i < 4 ? r0[i] : r1[i - 4];
-            r.k[i] = buf_load16(krs, row * kss + l16 * 16);
-            r.v[i] = buf_load16(vrs, row * vss + l16 * 16);
+            vr[i] = buf_load16(vrs, (kSameRows ? row : row * vss) + l16 * 16);
         }
     };
-    const int wrow = lane >> 4;   // row within each group of 4 entries
-    auto stage = [&](const Rows& r) {
+    auto transpose = [&](const u32x4_t (&r)[4], u32x4_t (&o)[4], int d) {
+        uint32_t a[4], b[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            *reinterpret_cast<u32x4_t*>(kl + (4 * i + wrow) * kSpKRow + l16 * 16) = r.k[i];
-            *reinterpret_cast<u32x4_t*>(vl + (4 * i + wrow) * kSpVRow + l16 * 16) = r.v[i];
-        }
+        for (int i = 0; i < 4; ++i) a[i] = r[i][d], b[i] = r[i][d + 1];
+        sp_transpose_quad(a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3], 0xAAAAAAAAAAAAAAAAull, 0xCCCCCCCCCCCCCCCCull);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i][d] = a[i], o[i][d + 1] = b[i];
     };
-    // A operand (K) of tile tt, k-step ks: lane (key l16, group g) reads dims
-    // 32*ks + 8g .. +7 of entry 16tt + l16.
-    const unsigned char* krd = kl + l16 * kSpKRow + g * 16;
+    auto stage_v = [&]() {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(tile + (8 * g + i) * kSpRow + l16 * 16) = vr[i];
+    };
     // Transposed V reads: lane (l16, g) of half kh supplies entry 16kh + 4g + l16/4,
     // dims 16dt + 4*(l16 % 4) .. +3, i.e. chunk 2dt + (l16/2) % 2, half l16 % 2.
-    const unsigned char* vrd = vl + (4 * g + (l16 >> 2)) * kSpVRow + ((l16 >> 1) & 1) * 16 + (l16 & 1) * 8;
+    const unsigned char* vrd = tile + (4 * g + (l16 >> 2)) * kSpRow + ((l16 >> 1) & 1) * 16 + (l16 & 1) * 8;
 
     const float c = p.scale_log2;
     float m_run = -INFINITY;   // running max (log2 units) of head l16
@@ -244,40 +264,11 @@ __global__ __launch_bounds__(kSpWaves * kWave, 2) void sparse_prefill_kernel(Spa
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) oacc[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    // One step on the staged entries.  S^T C layout: lane (head l16, group g)
-    // register r of tile tt = entry 16tt + 4g + r.
-    auto compute = [&](uint32_t mask) {
-        f32x4_t s[2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            s[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const bf16x8_t ka = *reinterpret_cast<const bf16x8_t*>(krd + tt * 16 * kSpKRow + ks * 64);
-                s[tt] = mfma16(ka, qop[ks], s[tt]);
-            }
-        }
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const bool ok = (mask >> (16 * tt + 4 * g + r)) & 1u;
-                s[tt][r] = ok ? s[tt][r] : -INFINITY;
-                tmax = fmaxf(tmax, s[tt][r]);
-            }
-        tmax = half_max(xor_max(tmax, 16)) * c;
-        if (__builtin_amdgcn_ballot_w64(tmax > m_run + kSpRescaleSlack) != 0) {
-            const float m_new = fmaxf(m_run, tmax);
-            const float m_new_use = (m_new == -INFINITY) ? 0.f : m_new;
-            const float alpha = fast_exp2(m_use - m_new_use);
-            l_run *= alpha;
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt) oacc[dt] *= alpha;
-            m_run = m_new;
-            m_use = m_new_use;
-        }
-        bf16x8_t pop;
+    // S^T C layout: lane (head l16, group g) register r of tile tt = tile row
+    // 16tt + 4g + r, the step's entry of that number.
+    f32x4_t s[2];
+    bf16x8_t pop;
+    auto softmax_p = [&]() -> float {
         float psum = 0.f;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
@@ -287,102 +278,108 @@ __global__ __launch_bounds__(kSpWaves * kWave, 2) void sparse_prefill_kernel(Spa
                 psum += pv;
                 pop[tt * 4 + r] = (__bf16)pv;
             }
-        l_run += psum;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-            const bf16x4_t lo = lds_read_tr16(reinterpret_cast<const __bf16*>(vrd + dt * 32));
-            const bf16x4_t hi = lds_read_tr16(reinterpret_cast<const __bf16*>(vrd + 16 * kSpVRow + dt * 32));
-            oacc[dt] = mfma16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pop, oacc[dt]);
-        }
+        return psum;
     };
-
-    // Step t: its rows (gathered two steps earlier) are staged into LDS, then
-    // step t + 2's rows are gathered into the freed register set while step t
-    // is computed.
-    if constexpr (kSorted) {
-        // The whole list (at most 512 entries) in ascending key order, unusable
-        // entries last: every wave walks the keys of its prefix from low to high
-        // at about the same pace as the other waves of its XCD, whose lists
-        // overlap, so a row one wave fetches is often still in L2 when another
-        // needs it (at the reference's shape 634 -> 477 us for pre-sorted lists
-        // against list order).  The order of the sum changes by rounding only.
-        // Lane l holds sorted entries 8l .. 8l+7; a step's 32 entries are lanes
-        // 4t .. 4t+3.  Only steps holding usable entries run.
+    for (int c0 = 0; c0 < p.nsparse; c0 += kSpList) {
+        // Up to 512 entries, the usable ones first and window by window
+        // (entries of a window in list order of their slots; deterministic).  The
+        // order of the sum changes by rounding only.
         int x[8];
         {
-            const u32x4_t a0 = buf_load16(irs, (uint32_t)lane * 32);
-            const u32x4_t a1 = buf_load16(irs, (uint32_t)lane * 32 + 16);
+            const u32x4_t a0 = buf_load16(irs, (uint32_t)(c0 + 8 * lane) * 4);
+            const u32x4_t a1 = buf_load16(irs, (uint32_t)(c0 + 8 * lane) * 4 + 16);
+            const int lim = p.causal ? min(pos + 1, p.skv) : p.skv;
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
                 const int jj = (int)(r < 4 ? a0[r] : a1[r - 4]);
-                const bool ok = 8 * lane + r < p.nsparse && jj >= 0 && jj < p.skv && (!p.causal || jj <= pos);
-                x[r] = ok ? jj : INT_MAX;
+                const bool ok = c0 + 8 * lane + r < p.nsparse && jj >= 0 && jj < lim;
+                x[r] = ok ? jj : -1;
             }
         }
-        sp_sort512(x, lane);
-        int n_valid = 0;
+        int at[8], n_valid = 0;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) n_valid += __builtin_popcountll(__builtin_amdgcn_ballot_w64(x[r] != INT_MAX));
-        const int steps = (n_valid + 2 * kSpStep - 1) / (2 * kSpStep) * 2;   // even
-        // rows of step t into the index area (lane l then finds the rows of
-        // entries 4i + l/16 in 8 consecutive words); unusable entries read row 0
-        auto post = [&](int t) {
-            if ((lane >> 2) == t) {
-                const int q = lane & 3;
+        for (int r = 0; r < 8; ++r) at[r] = kSpList;   // unusable: dropped
+        for (int w = 0; w < p.n_windows; ++w) {
 #pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const int e = 8 * q + r;
-                    il[(e & 3) * 8 + (e >> 2)] = x[r] == INT_MAX ? 0 : x[r];
-                }
+            for (int r = 0; r < 8; ++r) {
+                const bool in = (x[r] >> p.window_shift) == w;
+                const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+                const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, n_valid));
+                at[r] = in ? rank : at[r];
+                n_valid += __builtin_popcountll(m);
             }
-        };
-        auto step_mask = [&](int t) -> uint32_t {
-            const int nv = min(max(n_valid - t * kSpStep, 0), kSpStep);
-            return nv == kSpStep ? 0xffffffffu : ((1u << nv) - 1u);
-        };
-        post(0);
-        issue(ra);
-        post(1);
-        issue(rb);
-        for (int t = 0; t < steps; t += 2) {
-            stage(ra);
-            post(t + 2);
-            issue(ra);
-            compute(step_mask(t));
-            stage(rb);
-            post(t + 3);
-            issue(rb);
-            compute(step_mask(t + 1));
         }
-    } else {
-    // Index lists are loaded a step before their rows are
-    // gathered and before the rows in front of them, so waiting for a list never
-    // waits for rows.  Steps past nsparse are fully masked (their gathers read
-    // row 0 and are never used); n_steps is even, so the two register sets
-    // alternate without copies.
-    // One index load per loop trip, issued before the rows behind it.
-    int j = load_pair(0);
-    uint64_t mcur = pair_mask(0, j);
-    post_rows(j, mcur, 0);
-    issue(ra);
-    int jn = load_pair(2);
-    post_rows(j, mcur, 1);
-    issue(rb);
-    for (int t = 0; t < p.n_steps; t += 2) {
-        stage(ra);
-        const uint64_t mnext = pair_mask(t + 2, jn);
-        post_rows(jn, mnext, 0);
-        issue(ra);
-        compute((uint32_t)mcur);
-
-        stage(rb);
-        j = jn;
-        jn = load_pair(t + 4);
-        post_rows(j, mnext, 1);
-        issue(rb);
-        compute((uint32_t)(mcur >> 32));
-        mcur = mnext;
-    }
+        if (n_valid == 0) continue;
+        // (the last step's unused entries read row 0 and are masked)
+        {
+            int4* w = reinterpret_cast<int4*>(il + 8 * lane);
+            w[0] = w[1] = make_int4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 8; ++r) il[at[r]] = kSameRows ? (int)((uint32_t)x[r] * kss) : x[r];
+        const int steps = (n_valid + kSpStep - 1) / kSpStep;
+        issue_k(0);
+        issue_v(0);
+        for (int t = 0; t < steps; ++t) {
+            const bool more = t + 1 < steps;
+            u32x4_t kt[2][4];
+            u32x4_t(&ka)[2][4] = kPerSimd == 2 ? kt : kr;   // (three waves: in place, no registers to spare)
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int d = 0; d < 4; d += 2) transpose(kr[tt], ka[tt], d);
+            if constexpr (kPerSimd == 2) {
+                if (more) issue_k(t + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                s[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) s[tt] = mfma16(as_bf16x8(ka[tt][ks]), qop[ks], s[tt]);
+            }
+            if constexpr (kPerSimd == 3) {
+                if (more) issue_k(t + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            stage_v();
+            if (more) issue_v(t + 1);
+            const int nv = n_valid - t * kSpStep;
+            if (nv < kSpStep) {
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[tt][r] = 16 * tt + 4 * g + r < nv ? s[tt][r] : -INFINITY;
+            }
+            // P against the max so far; the max moves only when it must: at the
+            // first step, and when a lane's P sums to more than kSpMaxP (bf16's
+            // relative precision does not depend on P's size).
+            float lt = softmax_p();
+            if (__builtin_amdgcn_ballot_w64(m_run == -INFINITY || !(lt <= kSpMaxP)) != 0) {
+                float tmax = -INFINITY;
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[tt][r]);
+                tmax = half_max(xor_max(tmax, 16)) * c;
+                const float m_new = fmaxf(m_run, tmax);
+                const float m_new_use = (m_new == -INFINITY) ? 0.f : m_new;
+                const float alpha = fast_exp2(m_use - m_new_use);
+                l_run *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < 8; ++dt) oacc[dt] *= alpha;
+                m_run = m_new;
+                m_use = m_new_use;
+                lt = softmax_p();
+            }
+            l_run += lt;
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+                const bf16x4_t lo = lds_read_tr16(reinterpret_cast<const __bf16*>(vrd + dt * 32));
+                const bf16x4_t hi = lds_read_tr16(reinterpret_cast<const __bf16*>(vrd + 16 * kSpRow + dt * 32));
+                oacc[dt] = mfma16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pop, oacc[dt]);
+            }
+        }
     }
 
     // Row sums over the four lane groups; then O and the LSE of head l16.
@@ -445,20 +442,32 @@ extern "C" int fgqa_sparse_prefill_bf16(const fgqa_sparse_prefill_args* a, void*
     p.nsparse = a->num_sparse_kv;
     p.causal = a->causal ? 1 : 0;
     p.n_hg = (int)ceil_div(p.group, 16);
-    const int steps = (int)ceil_div(p.nsparse, kSpStep);
-    p.n_steps = steps + (steps & 1);
     p.n_items = (int64_t)p.batch * p.hkv * p.sq * p.n_hg;
+    p.div_hg = make_fast_div(p.n_hg);
+    p.div_sq = make_fast_div(p.sq);
+    p.div_hkv = make_fast_div(p.hkv);
+    int shift = 31;
+    if (p.skv > kSpNoWindows) {
+        const int most = std::max(std::min(p.nsparse, kSpList) / kSpStep, 1);
+        for (shift = kSpWindowLog2; ((p.skv - 1) >> shift) >= most;) ++shift;
+    }
+    p.window_shift = shift;
+    p.n_windows = p.skv > 0 ? ((p.skv - 1) >> shift) + 1 : 0;
     p.scale_log2 = fabsf(a->scale) * kLog2e;
     p.q_sign = (a->scale < 0.f) ? 0x80008000u : 0u;
 
     const int64_t blocks = ceil_div(p.n_items, kSpWaves);
     if (blocks >= ((int64_t)1 << 31)) return FGQA_ERR_UNSUPPORTED;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    // lists of at most 512 entries are taken in key order
-    if (p.nsparse <= 512)
-        hipLaunchKernelGGL(sparse_prefill_kernel<true>, dim3((unsigned)blocks), dim3(kSpWaves * kWave), 0, s, p);
-    else
-        hipLaunchKernelGGL(sparse_prefill_kernel<false>, dim3((unsigned)blocks), dim3(kSpWaves * kWave), 0, s, p);
+    const dim3 grid((unsigned)blocks), threads(kSpWaves * kWave);
+    const int cus = device_cu_count();
+    if (cus <= 0) return FGQA_ERR_HIP;
+    const bool few = p.skv > kSpManyKeys || blocks <= 2 * cus;
+    const bool same = p.k_ss == p.v_ss;
+    if (few && same) hipLaunchKernelGGL((sparse_prefill_kernel<true, 2>), grid, threads, 0, s, p);
+    else if (few) hipLaunchKernelGGL((sparse_prefill_kernel<false, 2>), grid, threads, 0, s, p);
+    else if (same) hipLaunchKernelGGL((sparse_prefill_kernel<true, 3>), grid, threads, 0, s, p);
+    else hipLaunchKernelGGL((sparse_prefill_kernel<false, 3>), grid, threads, 0, s, p);
     if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
     return FGQA_OK;
 }
