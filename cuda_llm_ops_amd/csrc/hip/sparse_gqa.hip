@@ -110,7 +110,9 @@ __device__ __forceinline__ int64_t sp_block_first_item(int64_t nblocks) {
 // a time: each of the 16 moves takes the neighbour's register through DPP and
 // keeps or replaces by a lane mask (v_cndmask with a DPP source; the masks go
 // through vcc).  A DPP read needs two wait states after a VALU write of its
-// register: the s_nop covers what comes before, the order of the moves the rest.
+// register: the first s_nop covers what comes before, the order of the moves the
+// rest.  The last one keeps an MFMA that follows two states behind the moves (the
+// compiler counts no wait states around inline asm).
 __device__ __forceinline__ void sp_transpose_quad(uint32_t& a0, uint32_t& a1, uint32_t& a2, uint32_t& a3,
                                                   uint32_t& b0, uint32_t& b1, uint32_t& b2, uint32_t& b3,
                                                   uint64_t bit0, uint64_t bit1) {
@@ -135,7 +137,8 @@ __device__ __forceinline__ void sp_transpose_quad(uint32_t& a0, uint32_t& a1, ui
         "v_cndmask_b32_dpp %[a2], %[t0], %[t2], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
         "v_cndmask_b32_dpp %[a3], %[t1], %[t3], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
         "v_cndmask_b32_dpp %[b2], %[u0], %[u2], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-        "v_cndmask_b32_dpp %[b3], %[u1], %[u3], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+        "v_cndmask_b32_dpp %[b3], %[u1], %[u3], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1"
         : [a0] "+v"(a0), [a1] "+v"(a1), [a2] "+v"(a2), [a3] "+v"(a3), [b0] "+v"(b0), [b1] "+v"(b1), [b2] "+v"(b2),
           [b3] "+v"(b3), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3), [u0] "=&v"(u0),
           [u1] "=&v"(u1), [u2] "=&v"(u2), [u3] "=&v"(u3)
