@@ -285,7 +285,7 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
     };
     for (int c0 = 0; c0 < p.nsparse; c0 += kSpList) {
         // Up to 512 entries, the usable ones first and window by window
-        // (entries of a window in list order of their slots; deterministic).  The
+        // (a fixed order, by slot modulo 8 and then lane, in a window).  The
         // order of the sum changes by rounding only.
         int x[8];
         {

@@ -234,7 +234,10 @@ int fgqa_decode_paged(const fgqa_decode_paged_args* args, void* stream);
  *           to a power of two (src/python/Triton/flash_gqa_kernel.py:
  *           266-269); zero columns add nothing to q.k^T.  Those copies are
  *           made element by element, so such calls need neither 16-byte
- *           alignment nor strides in multiples of 8.  Head dims above 256
+ *           alignment nor strides in multiples of 8.  (Pairs with both dims
+ *           up to 64 and multiples of 8, with aligned tensors and strides in
+ *           multiples of 8, run kernels built for 64 in place, except
+ *           FGQA_KERNEL_TALL.)  Head dims above 256
  *           return FGQA_ERR_UNSUPPORTED, and so do a window or sink with
  *           head_dim 192 and FGQA_KERNEL_SPLIT / _WIDE / _TALL with q/k
  *           padded to 256.
