@@ -6,6 +6,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 namespace fgqa {
 namespace plan {
 
@@ -355,8 +357,13 @@ bool wide_on_pairs(const fgqa_prefill_args* a, int cus) {
 
 bool tall_on_pairs(const fgqa_prefill_args* a, int cus) { return a->causal && wide_on_pairs(a, cus); }
 
+// The most keys that a query row sees.
+static int64_t longest_row(const fgqa_prefill_args* a) {
+    return a->causal ? std::min(a->seqlen_q, a->seqlen_kv) : a->seqlen_kv;
+}
+
 // AUTO for the kernels built for head dim 64 without a window or sink, by the
-// 128-row units and the query rows S (a unit's steps).  Two units share a CU in
+// 128-row units and the keys S of the longest row (a unit's steps).  Two units share a CU in
 // the whole-range kernel there (half the LDS and registers of head dim 128's),
 // so it wins as soon as the grid gives every CU more than one unit, where the
 // split kernel needs a second round.  Measured on 430 grids (Hq/Hkv 16/1, 32/8,
@@ -373,8 +380,8 @@ bool tall_on_pairs(const fgqa_prefill_args* a, int cus) { return a->causal && wi
 //    60 / 49 / 50, 1024 units 85 / 95 / 82; S = 4096 full, 512 units 86 / 91 / 79.
 //  - the rest: whole.  S = 1280 causal, 1280 units 38 / 57 / 49.
 static int choice_native64(const fgqa_prefill_args* a, int64_t units, int64_t cus) {
-    const int64_t s = a->seqlen_q;
-    if (a->seqlen_kv <= 448) return FGQA_KERNEL_WHOLE;
+    const int64_t s = longest_row(a);
+    if (s <= 448) return FGQA_KERNEL_WHOLE;
     if (!a->causal) {
         if (units <= cus) return FGQA_KERNEL_SPLIT;
         return s >= 1536 && units <= 2 * cus ? FGQA_KERNEL_WIDE : FGQA_KERNEL_WHOLE;
@@ -388,7 +395,9 @@ static int choice_native64(const fgqa_prefill_args* a, int64_t units, int64_t cu
 // AUTO's short sequences and full (non-causal) grids at head dim 128 without a
 // window or sink; AUTO: none of them, the general lines of prefill_choice.
 // Measured on 780 grids (as above, also Hq/Hkv 28/4 and 16/2, B up to 8; us,
-// whole / split / wide):
+// whole / split / wide), and on 380 with Sq != Skv, where the longest row's keys
+// stand for S (causal, Sq = 64, Skv = 2048, 32 units: 6.7 / 8.8 / 10.6; Sq = 4096,
+// Skv = 256, 512 units: 16.7 / 19.8 / 18.1):
 //  - a unit per CU or fewer: the split kernel halves a unit's steps but pays
 //    for the merge; up to 5 tiles of 64 keys, or 7 (4 + 3), there is nothing to
 //    gain.  S = 192, 128 units 8.4 / 10.0 / 13.2; S = 300, 80 units 10.4 / 11.4 /
@@ -410,7 +419,7 @@ static int choice_native64(const fgqa_prefill_args* a, int64_t units, int64_t cu
 //    fgqa_prefill_kernel_choice has always reported for them (64 per CU: 16.0
 //    ms against 14.1).
 static int choice_short_or_full(const fgqa_prefill_args* a, int64_t units, int64_t cus) {
-    const int64_t s = a->seqlen_q, tiles = ceil_div(a->seqlen_kv, 64), wu = wide_units(a);
+    const int64_t s = longest_row(a), tiles = ceil_div(s, 64), wu = wide_units(a);
     if (units <= cus) return tiles <= 5 || tiles == 7 ? FGQA_KERNEL_WHOLE : FGQA_KERNEL_AUTO;
     if (a->causal) {
         if (units > 2 * cus) return 200 * wu > 108 * units ? FGQA_KERNEL_WHOLE : FGQA_KERNEL_AUTO;

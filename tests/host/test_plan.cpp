@@ -413,6 +413,19 @@ static void test_prefill_choice_lines() {
         const fgqa_prefill_args a = prefill_args(l.B, l.S, l.hq, l.hkv, l.causal);
         CHECK(plan::prefill_choice(&a, kCus) == l.want);
     }
+    // Sq != Skv: the longest row's keys count
+    for (const int d : {64, 128}) {
+        fgqa_prefill_args a = prefill_args(4, 64, 16, 1, true);
+        a.head_dim = a.head_dim_v = d;
+        a.seqlen_kv = 4096;
+        CHECK(plan::prefill_choice(&a, kCus) == FGQA_KERNEL_WHOLE);
+        a.causal = 0;
+        CHECK(plan::prefill_choice(&a, kCus) == FGQA_KERNEL_SPLIT);
+        a = prefill_args(1, 4096, 16, 1, true);
+        a.head_dim = a.head_dim_v = d;
+        a.seqlen_kv = 256;
+        CHECK(plan::prefill_choice(&a, kCus) == FGQA_KERNEL_WHOLE);
+    }
     for (const int hq : {16, 8, 6, 3})
         for (const int hkv : {1, 2, 8})
             for (int S = 1; S < 9000; S += 1 + S / 5)
