@@ -233,7 +233,7 @@ int fgqa_decode_paged(const fgqa_decode_paged_args* args, void* stream);
  *           out, as the reference's Triton launcher pads its head-dim blocks
  *           to a power of two (src/python/Triton/flash_gqa_kernel.py:
  *           266-269); zero columns add nothing to q.k^T.  Those copies are
- *           made element by element, so such calls need neither 16-byte
+ *           made element by element where need be, so such calls need neither 16-byte
  *           alignment nor strides in multiples of 8.  (Pairs with both dims
  *           up to 64 and multiples of 8, with aligned tensors and strides in
  *           multiples of 8, run kernels built for 64 in place, except
