@@ -1,6 +1,8 @@
 // Host-side internals shared by the flash-GQA translation units.
 #pragma once
 
+#include <float.h>
+
 #include <mutex>
 
 #include <hip/hip_runtime.h>
@@ -11,6 +13,12 @@
 #include "../host/fgqa_plan.h"   // aligned16, ceil_div and the host-only validation / planning
 
 namespace fgqa {
+
+// The scale (in log2 units, >= 0) that a kernel multiplies its scores by, -inf
+// where masked.  0 becomes the smallest normal number: -inf stays -inf (times 0
+// it would be NaN), and a visible score of ordinary size comes out as 0 to
+// within fp32's resolution of exp2 and of the LSE.
+inline float score_scale(float c) { return c < FLT_MIN ? FLT_MIN : c; }
 
 // Compute units of the current device (queried once per device, then cached).
 // Returns 0 when the device cannot be queried.

@@ -1473,7 +1473,7 @@ int prefill_launch(const fgqa_prefill_args* a, hipStream_t s) {
     p.div_streams = make_fast_div(p.n_streams);
     p.div_hgroups = make_fast_div(p.n_hgroups);
     p.div_hkv = make_fast_div(p.hkv);
-    p.scale_log2 = fabsf(a->scale) * kLog2e;
+    p.scale_log2 = score_scale(fabsf(a->scale) * kLog2e);
     p.q_sign = (a->scale < 0.f) ? 0x80008000u : 0u;
     p.window = a->window_size;
     p.sink = a->sink;
