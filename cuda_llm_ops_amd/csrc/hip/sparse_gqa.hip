@@ -456,7 +456,7 @@ extern "C" int fgqa_sparse_prefill_bf16(const fgqa_sparse_prefill_args* a, void*
     }
     p.window_shift = shift;
     p.n_windows = p.skv > 0 ? ((p.skv - 1) >> shift) + 1 : 0;
-    p.scale_log2 = fabsf(a->scale) * kLog2e;
+    p.scale_log2 = score_scale(fabsf(a->scale) * kLog2e);
     p.q_sign = (a->scale < 0.f) ? 0x80008000u : 0u;
 
     const int64_t blocks = ceil_div(p.n_items, kSpWaves);
