@@ -868,7 +868,7 @@ int backward_launch(const fgqa_prefill_backward_args* a, hipStream_t s) {
     p.hkv = a->num_kv_heads;
     p.group = a->num_q_heads / a->num_kv_heads;
     p.causal = a->causal ? 1 : 0;
-    p.window = a->window_size;
+    p.window = plan::effective_window(a->window_size, a->seqlen_q);
     p.n_hsplit = pl.n_hsplit;
     p.hs = p.group / pl.n_hsplit;
     p.n_kvblocks = (int)ceil_div(p.skv, plan::kBackwardKvKeys);

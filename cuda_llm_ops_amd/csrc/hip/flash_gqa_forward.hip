@@ -1475,7 +1475,7 @@ int prefill_launch(const fgqa_prefill_args* a, hipStream_t s) {
     p.div_hkv = make_fast_div(p.hkv);
     p.scale_log2 = score_scale(fabsf(a->scale) * kLog2e);
     p.q_sign = (a->scale < 0.f) ? 0x80008000u : 0u;
-    p.window = a->window_size;
+    p.window = plan::effective_window(a->window_size, a->seqlen_q);
     p.sink = a->sink;
     p.dk8 = a->head_dim / 8;
     p.dv8 = (a->head_dim_v == 0 ? a->head_dim : a->head_dim_v) / 8;

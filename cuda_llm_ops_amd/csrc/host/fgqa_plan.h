@@ -26,6 +26,14 @@ constexpr int kHeadDim = 128;   // D (and Dv) of every kernel; MLA's Q/K head di
 // their tile-rounded ends stay far inside the kernels' 32-bit integers.
 constexpr int kMaxTokens = 1 << 30;
 
+// A sliding window as the kernels take it: one longer than the query rows hides
+// no causal key, and cut to their number it keeps the sums of a position and the
+// window inside 32 bits.
+inline int effective_window(int window, int seqlen_q) {
+    const int most = seqlen_q > 1 ? seqlen_q : 1;
+    return window < most ? window : most;
+}
+
 // ---------------------------------------------------------------- decode
 constexpr int kDecodeStepRound = 128;     // tokens of one pass of a decode workgroup's 4 waves
 constexpr int kDecodeMaxAutoChunk = 4096; // longest split the planner picks by itself

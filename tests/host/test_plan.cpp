@@ -437,6 +437,19 @@ static void test_prefill_choice_lines() {
                 }
 }
 
+// The window the kernels get: never longer than the query rows, never 0 for a
+// window that was given, and no window stays none.
+static void test_effective_window() {
+    const int huge = 2147483647;
+    for (const int sq : {0, 1, 2, 300, 1 << 30}) {
+        CHECK(plan::effective_window(0, sq) == 0);
+        CHECK(plan::effective_window(1, sq) == 1);
+        CHECK(plan::effective_window(huge, sq) == (sq > 0 ? sq : 1));
+        CHECK(plan::effective_window(sq, sq) == (sq > 0 ? sq : 0));
+    }
+    CHECK(plan::effective_window(299, 300) == 299 && plan::effective_window(301, 300) == 300);
+}
+
 static void test_prefill_rejections() {
     const fgqa_prefill_args a = prefill_args(1, 4096, 16, 1, true);
     fgqa_prefill_args b = a;
@@ -974,6 +987,7 @@ int main() {
     test_paged();
     test_prefill_known_shapes();
     test_prefill_choice_lines();
+    test_effective_window();
     test_prefill_rejections();
     test_prefill_padded_head_dims();
     test_backward();
