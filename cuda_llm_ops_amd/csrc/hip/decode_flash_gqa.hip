@@ -874,6 +874,31 @@ int32_t* carve_workspace(const DecodePlan& plan, void* ws, DecodeParams* p) {
     return work;
 }
 
+// The workspace of a call that needs one: the caller's (*ws, bytes), or for
+// null and 0 the library's buffer, whose lock is then held.  Sets *ws, and the
+// plan's form to what it holds.  A capture cannot grow the library's buffer: it
+// takes the list's form where the buffer is large enough for that alone.
+int take_workspace(DecodePlan* plan, size_t bytes, hipStream_t s, std::unique_lock<std::mutex>* lock, void** ws) {
+    if (*ws == nullptr && bytes == 0) {
+        *lock = workspace_lock();
+        size_t want = plan->ws_bytes;
+        const size_t have = internal_workspace_size();
+        if (have < want && have >= plan->least_bytes) {
+            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+            if (capture != hipStreamCaptureStatusNone) want = plan->least_bytes;
+        }
+        plan::fit_workspace(plan, want);
+        int st = FGQA_OK;
+        *ws = internal_workspace(want, &st);
+        return st;
+    }
+    if (*ws == nullptr || bytes < plan->least_bytes) return FGQA_ERR_WORKSPACE;
+    if (!aligned16(*ws)) return FGQA_ERR_UNSUPPORTED;
+    plan::fit_workspace(plan, bytes);
+    return FGQA_OK;
+}
+
 // The split plan of a validated call on the current device.
 int plan_on_device(const DecodeShape& shape, DecodePlan* pl) {
     const int cus = plan::decode_needs_cus(shape) ? device_cu_count() : 0;
@@ -978,6 +1003,7 @@ int decode_run(const fgqa_decode_args* a, void* stream, bool noalloc) {
     p.chunk = plan.chunk;
     p.scale_log2 = a->scale * kLog2e;
 
+    const hipStream_t s = static_cast<hipStream_t>(stream);
     int32_t* work = nullptr;
     std::unique_lock<std::mutex> ws_lock;   // held through the launches when the library's buffer is used
     if (plan.ws_bytes > 0) {
@@ -988,19 +1014,12 @@ int decode_run(const fgqa_decode_args* a, void* stream, bool noalloc) {
             if (plan.ws_bytes > kNoAllocScratchBytes) return FGQA_ERR_WORKSPACE;
             ws = noalloc_scratch(&st);
             if (ws == nullptr) return st;
-        } else if (ws == nullptr && a->workspace_bytes == 0) {
-            ws_lock = workspace_lock();
-            ws = internal_workspace(plan.ws_bytes, &st);
-            if (st != FGQA_OK) return st;
-        } else if (ws == nullptr || a->workspace_bytes < plan.ws_bytes) {
-            return FGQA_ERR_WORKSPACE;
-        } else if (!aligned16(ws)) {
-            return FGQA_ERR_UNSUPPORTED;
+        } else if (st = take_workspace(&plan, a->workspace_bytes, s, &ws_lock, &ws); st != FGQA_OK) {
+            return st;
         }
         work = carve_workspace(plan, ws, &p);
     }
 
-    hipStream_t s = static_cast<hipStream_t>(stream);
     if (a->max_seqlen == 0) {
         // Every sequence is empty: the combine writes O = 0, lse = -inf.
         launch_combine<false>(p, 1, s);
@@ -1096,23 +1115,16 @@ extern "C" int fgqa_decode_paged(const fgqa_decode_paged_args* a, void* stream) 
     p.num_pages = a->num_pages;
     p.v_scale = a->v_scale;
 
+    const hipStream_t s = static_cast<hipStream_t>(stream);
     int32_t* work = nullptr;
     std::unique_lock<std::mutex> ws_lock;   // held through the launches when the library's buffer is used
     if (plan.ws_bytes > 0) {
         void* ws = a->workspace;
-        if (ws == nullptr && a->workspace_bytes == 0) {
-            ws_lock = workspace_lock();
-            ws = internal_workspace(plan.ws_bytes, &st);
-            if (st != FGQA_OK) return st;
-        } else if (ws == nullptr || a->workspace_bytes < plan.ws_bytes) {
-            return FGQA_ERR_WORKSPACE;
-        } else if (!aligned16(ws)) {
-            return FGQA_ERR_UNSUPPORTED;
-        }
+        st = take_workspace(&plan, a->workspace_bytes, s, &ws_lock, &ws);
+        if (st != FGQA_OK) return st;
         work = carve_workspace(plan, ws, &p);
     }
 
-    hipStream_t s = static_cast<hipStream_t>(stream);
     if (a->max_seqlen == 0) {
         launch_combine<false>(p, 1, s);
     } else {

@@ -31,6 +31,8 @@ int device_cu_count();
 // and sets *status on failure.
 std::unique_lock<std::mutex> workspace_lock();
 void* internal_workspace(size_t bytes, int* status);
+// Its size on the current device so far (under the lock too).
+size_t internal_workspace_size();
 
 // Sets a kernel's dynamic-LDS limit once per device (the attribute is per
 // kernel and per device).  slot: a distinct small index per kernel.

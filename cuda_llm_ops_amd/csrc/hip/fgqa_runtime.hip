@@ -45,6 +45,11 @@ int set_kernel_smem_once(int slot, const void* fn, int bytes) {
 
 std::unique_lock<std::mutex> workspace_lock() { return std::unique_lock<std::mutex>(g_ws_mutex); }
 
+size_t internal_workspace_size() {
+    int dev = 0;
+    return hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices ? 0 : g_ws_bytes[dev];
+}
+
 void* internal_workspace(size_t bytes, int* status) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) {

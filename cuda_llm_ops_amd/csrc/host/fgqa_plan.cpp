@@ -142,11 +142,13 @@ int plan_decode(const DecodeShape& a, int cus, DecodePlan* plan) {
     plan->part_o_bytes = round256(part_o);
     plan->part_ml_bytes = round256(part_ml);
     plan->ws_bytes = plan->part_o_bytes + plan->part_ml_bytes + (size_t)list;
+    plan->least_bytes = plan->ws_bytes;
     plan->teams = 0;
     plan->team_ml_off = plan->team_prefix_off = 0;
     if (plan->list && a.split_tokens == 0 && a.num_kv_heads <= kDecodeItemSlots) {
-        // (the list's formula stays the least workspace, so that which calls
-        // fit a given scratch does not depend on how the batch is shared out)
+        // (the list's size stays the least that a caller's scratch needs, so
+        // that which calls fit a scratch does not depend on how the batch is
+        // shared out)
         plan->teams = kDecodeItemSlots / a.num_kv_heads;
         const i128 rows = (i128)2 * plan->teams * a.num_q_heads;
         plan->team_ml_off = round256(rows * kHeadDim * 4);
@@ -155,6 +157,10 @@ int plan_decode(const DecodeShape& a, int cus, DecodePlan* plan) {
         if (need > plan->ws_bytes) plan->ws_bytes = need;
     }
     return FGQA_OK;
+}
+
+void fit_workspace(DecodePlan* plan, size_t bytes) {
+    if (bytes < plan->ws_bytes) plan->teams = 0;
 }
 
 int validate_paged(const fgqa_decode_paged_args* a) {

@@ -60,11 +60,18 @@ struct DecodePlan {
                           // teams (else 0)
     size_t part_o_bytes;  // fp32 partial O of every split (nsplit > 1)
     size_t part_ml_bytes; // their (max, sum)
-    size_t ws_bytes;      // the workspace: partials, then the list (1 + batch * nsplit int32)
+    size_t ws_bytes;      // the workspace to ask for: partials, then the list (1 + batch * nsplit int32); teams: at
+                          // least what they take
     // teams > 0: the workspace holds the partials of two items per team, their
-    // (max, sum) and the sequences' block prefix (batch + 1 int64) instead
+    // (max, sum) and the sequences' block prefix (batch + 1 int64) instead.
+    // One of least_bytes only (the list's size; ws_bytes without teams) is
+    // enough too: fit_workspace then takes the list.
+    size_t least_bytes;
     size_t team_ml_off, team_prefix_off;
 };
+
+// The plan's form that a workspace of `bytes` (at least least_bytes) holds.
+void fit_workspace(DecodePlan* plan, size_t bytes);
 
 int validate_decode(const fgqa_decode_args* a);
 int validate_decode_pointers(const fgqa_decode_args* a);

@@ -33,7 +33,7 @@ enum fgqa_status {
     FGQA_ERR_UNSUPPORTED = -2,      /* valid but not implemented: head_dim, group size, alignment,
                                        sequence lengths above 2^30, grids of 2^31 workgroups or more,
                                        one sequence's K/V/Q span reaching 2 GiB */
-    FGQA_ERR_WORKSPACE = -3,        /* caller workspace smaller than fgqa_decode_workspace_bytes */
+    FGQA_ERR_WORKSPACE = -3,        /* caller workspace smaller than the call needs */
     FGQA_ERR_HIP = -4               /* a HIP runtime call or kernel launch failed */
 };
 
@@ -95,6 +95,13 @@ enum fgqa_kernel_choice {
  *            that share that buffer must not run at the same time on the GPU:
  *            concurrent calls on different streams of one device each pass
  *            their own workspace.  (Host threads may call concurrently.)
+ *            Ragged calls (seqlens, split_tokens 0) share the batch's tokens
+ *            out evenly over the chip, which takes up to 8.5 MB and 8 bytes
+ *            per sequence; they also accept a smaller workspace, down to what
+ *            4096-token splits take (n = ceil(max_seqlen / 4096): for n > 1,
+ *            B * Hq * n * 520 bytes with each of the two parts, of 512 and 8,
+ *            rounded up to 256; and 4 * (1 + B * n) bytes), and then run
+ *            those, more slowly.
  */
 typedef struct fgqa_decode_args {
     const void* q;

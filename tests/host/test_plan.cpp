@@ -127,6 +127,38 @@ static void test_decode_known_shapes() {
     }
 }
 
+// Ragged batches shared out over teams still run in a workspace of the list's
+// size, as the list, and in nothing less.
+static void test_decode_least_workspace() {
+    for (const int B : {1, 2, 8, 64, 1000})
+        for (const int S : {0, 1, 300, 4096, 4097, 32768})
+            for (const int hkv : {1, 3, 8, 512, 513}) {
+                fgqa_decode_args a = decode_args(B, S, 4 * hkv, hkv);
+                int32_t lens[1];
+                a.seqlens = lens;
+                plan::DecodePlan pl;
+                CHECK(plan::plan_decode(plan::decode_shape(&a), 0, &pl) == FGQA_OK);
+                CHECK(pl.list && (pl.teams > 0) == (hkv <= 512));
+                const size_t n = (size_t)(S > 4096 ? (S + 4095) / 4096 : 1);
+                const size_t slots = (size_t)B * a.num_q_heads * n;
+                const size_t part = n > 1 ? (slots * 512 + 255) / 256 * 256 + (slots * 8 + 255) / 256 * 256 : 0;
+                CHECK(pl.least_bytes == part + 4 * (1 + B * n) && pl.least_bytes <= pl.ws_bytes);
+                plan::DecodePlan q = pl;
+                plan::fit_workspace(&q, pl.ws_bytes);
+                CHECK(q.teams == pl.teams);
+                if (pl.teams > 0) {
+                    CHECK(pl.ws_bytes >= pl.team_prefix_off + 8 * ((size_t)B + 1));
+                    plan::fit_workspace(&q, pl.ws_bytes - 1);
+                    CHECK(q.teams == 0);
+                }
+            }
+    // uniform batches and given split lengths: all of it is needed
+    fgqa_decode_args a = decode_args(2, 4096, 16, 2);
+    plan::DecodePlan pl;
+    CHECK(plan::plan_decode(plan::decode_shape(&a), kCus, &pl) == FGQA_OK);
+    CHECK(pl.ws_bytes > 0 && pl.least_bytes == pl.ws_bytes);
+}
+
 static void test_decode_rejections() {
     fgqa_decode_args a = decode_args(2, 512, 16, 2);
     CHECK(plan::validate_decode(nullptr) == FGQA_ERR_INVALID_ARGUMENT);
@@ -982,6 +1014,7 @@ static void fuzz(unsigned seed, int rounds) {
 
 int main() {
     test_decode_known_shapes();
+    test_decode_least_workspace();
     test_decode_rejections();
     test_decode_extremes();
     test_paged();
