@@ -1323,8 +1323,8 @@ namespace {
 int prefill_launch(const fgqa_prefill_args* a, hipStream_t s);
 
 // Head dims the kernels are not built for (plan::prefill_padded).  Both up to
-// 64 and aligned (plan::prefill_native64): the kernels built for 64, on the
-// tensors themselves (the workspace bytes asked for stay those of the copies).
+// 64 and aligned (plan::prefill_native64), and O apart from the inputs: the
+// kernels built for 64, on the tensors themselves (the workspace bytes asked for stay those of the copies).
 // Else: pad, run the built kernels on the copies (once per 128 columns of V), unpad O.  The
 // copies live in the caller's workspace after the merge scratch, or with
 // none in the library's cached buffer (the merge scratch then being the
@@ -1338,7 +1338,7 @@ int prefill_padded_launch(const fgqa_prefill_args* a, hipStream_t s) {
     std::unique_lock<std::mutex> lock;
     unsigned char* base = nullptr;   // the copies: base + L.q .. base + L.total
     unsigned char* ws = static_cast<unsigned char*>(a->workspace);
-    const bool native = plan::prefill_native64(a);
+    const bool native = plan::prefill_native64(a) && !plan::prefill_output_meets_input(a);
     if (ws == nullptr && a->workspace_bytes == 0) {
         if (native) return prefill_launch(a, s);
         lock = workspace_lock();

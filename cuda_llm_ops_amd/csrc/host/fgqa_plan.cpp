@@ -239,6 +239,23 @@ bool prefill_native64(const fgqa_prefill_args* a) {
     return true;
 }
 
+bool prefill_output_meets_input(const fgqa_prefill_args* a) {
+    // first and last byte of rows of d elements at strides {b, s, h}
+    struct Range { i128 lo, hi; };
+    auto range = [](const void* p, int64_t b, int64_t s, int64_t h, const int64_t* st, int d) {
+        const i128 lo = (i128) reinterpret_cast<uintptr_t>(p);
+        return Range{lo, lo + 2 * ((i128)(b - 1) * st[0] + (i128)(s - 1) * st[1] + (i128)(h - 1) * st[2] + d) - 1};
+    };
+    const int dv = head_dim_v_of(a);
+    const Range o = range(a->o, a->batch, a->seqlen_q, a->num_q_heads, a->o_stride, dv);
+    const Range in[3] = {range(a->q, a->batch, a->seqlen_q, a->num_q_heads, a->q_stride, a->head_dim),
+                         range(a->k, a->batch, a->seqlen_kv, a->num_kv_heads, a->k_stride, a->head_dim),
+                         range(a->v, a->batch, a->seqlen_kv, a->num_kv_heads, a->v_stride, dv)};
+    for (int i = 0; i < 3; ++i)
+        if ((i == 0 || a->seqlen_kv > 0) && o.lo <= in[i].hi && in[i].lo <= o.hi) return true;
+    return false;
+}
+
 int padded_dk(const fgqa_prefill_args* a) {
     return a->head_dim <= kHeadDim ? kHeadDim : a->head_dim == 192 ? 192 : 256;
 }

@@ -113,6 +113,9 @@ bool prefill_padded(const fgqa_prefill_args* a);
 // the head dims read as zeros and are not written.  Same kernel shape, and the
 // same bits, as on the copies.
 bool prefill_native64(const fgqa_prefill_args* a);
+// O's bytes and those of Q, K or V may meet: such a call stays on the copies,
+// which are made before anything is written.
+bool prefill_output_meets_input(const fgqa_prefill_args* a);
 int padded_dk(const fgqa_prefill_args* a);
 int padded_dv(const fgqa_prefill_args* a);
 // The call on the copies (head dims padded_dk() and 128, V and O rows of

@@ -482,6 +482,35 @@ static void test_effective_window() {
     CHECK(plan::effective_window(299, 300) == 299 && plan::effective_window(301, 300) == 300);
 }
 
+// Where O's bytes may meet an input's: byte ranges, a byte on either side.
+static void test_prefill_output_meets_input() {
+    fgqa_prefill_args a = prefill_args(2, 100, 4, 4, true);
+    a.head_dim = a.head_dim_v = 64;
+    const int64_t st[3] = {100 * 4 * 64, 4 * 64, 64};
+    memcpy(a.q_stride, st, sizeof st);
+    memcpy(a.k_stride, st, sizeof st);
+    memcpy(a.v_stride, st, sizeof st);
+    memcpy(a.o_stride, st, sizeof st);
+    const uintptr_t bytes = 2 * 100 * 4 * 64 * 2, base = 1 << 24;
+    const void** in[3] = {&a.q, &a.k, &a.v};
+    for (int x = 0; x < 3; ++x) {
+        for (int y = 0; y < 3; ++y) *in[y] = reinterpret_cast<const void*>(base + (1 + (uintptr_t)y) * 4 * bytes);
+        const uintptr_t at = reinterpret_cast<uintptr_t>(*in[x]);
+        struct { uintptr_t o; bool meets; } const cases[] = {
+            {at, true}, {at + bytes - 2, true}, {at + bytes, false}, {at - bytes, false}, {at - bytes + 2, true}};
+        for (const auto& c : cases) {
+            a.o = reinterpret_cast<void*>(c.o);
+            CHECK(plan::prefill_output_meets_input(&a) == c.meets);
+        }
+    }
+    // heads of one row buffer side by side (q | o): their ranges meet
+    a.o = const_cast<char*>(static_cast<const char*>(a.q)) + 64 * 2;
+    CHECK(plan::prefill_output_meets_input(&a));
+    a.seqlen_kv = 0;   // no key rows: no bytes of K or V
+    a.o = const_cast<void*>(a.k);
+    CHECK(!plan::prefill_output_meets_input(&a));
+}
+
 static void test_prefill_rejections() {
     const fgqa_prefill_args a = prefill_args(1, 4096, 16, 1, true);
     fgqa_prefill_args b = a;
@@ -1021,6 +1050,7 @@ int main() {
     test_prefill_known_shapes();
     test_prefill_choice_lines();
     test_effective_window();
+    test_prefill_output_meets_input();
     test_prefill_rejections();
     test_prefill_padded_head_dims();
     test_backward();
