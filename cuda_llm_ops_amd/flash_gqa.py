@@ -421,6 +421,31 @@ def _new_prefill_workspace(nbytes, device):
     return ws
 
 
+def _span(p, st, b, s, h, d):
+    """First byte and end of rows of d bf16 elements at strides {b, s, h}."""
+    return p, p + 2 * ((b - 1) * st[0] + (s - 1) * st[1] + (h - 1) * st[2] + d)
+
+
+def _uses_no_scratch(a) -> bool:
+    """The call runs at a head dim up to 64 on the tensors themselves and merges
+    nothing, so the copies that the size query counts are not made: dims,
+    addresses and strides in multiples of 8 elements, O apart from the inputs
+    (else the library makes the copies), and no causal grid of at most 256 units
+    of 256 rows (others never merge)."""
+    dqk, dv = a.head_dim, a.head_dim_v or a.head_dim
+    if dqk > 64 or dv > 64 or (dqk | dv) & 7 or a.kernel == _lib.FGQA_KERNEL_TALL:
+        return False
+    if a.causal and a.batch * a.num_q_heads * a.seqlen_q <= 65536:
+        return False
+    if (a.q | a.k | a.v | a.o) & 15 or any(s & 7 for st in (a.q_stride, a.k_stride, a.v_stride, a.o_stride) for s in st):
+        return False
+    q_rows, kv_rows = (a.batch, a.seqlen_q, a.num_q_heads), (a.batch, a.seqlen_kv, a.num_kv_heads)
+    o0, o1 = _span(a.o, a.o_stride, *q_rows, dv)
+    spans = (_span(a.q, a.q_stride, *q_rows, dqk), _span(a.k, a.k_stride, *kv_rows, dqk),
+             _span(a.v, a.v_stride, *kv_rows, dv))
+    return all(hi <= o0 or o1 <= lo for lo, hi in spans)
+
+
 def _attach_prefill_workspace(a, device, own=False):
     """Sets `a`'s workspace for the kernel its call runs on this device: the
     current stream's cached one, or (own) a new one; None when the kernel
@@ -429,6 +454,9 @@ def _attach_prefill_workspace(a, device, own=False):
     _lib.check(_lib.lib().fgqa_prefill_workspace_bytes(ctypes.byref(a), ctypes.byref(n)),
                "fgqa_prefill_workspace_bytes")
     if n.value == 0:
+        return None
+    # (smaller ones are kept without a look: it would cost a short call a few us)
+    if n.value > 1 << 25 and _uses_no_scratch(a):
         return None
     if own:
         ws = _new_prefill_workspace(n.value, device)
