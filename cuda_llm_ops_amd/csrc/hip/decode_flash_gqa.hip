@@ -464,17 +464,41 @@ __global__ __launch_bounds__(kPair ? 2 * kDecThreads : kDecThreads) void decode_
 constexpr int kPlanThreads = 256;
 constexpr int kPlanSortMax = 1024;   // remainders kept in LDS and length-sorted up to this batch size
 
+// The value of the lane that DPP control kCtrl names, 0 where there is none or
+// the row is not in kRows.
+template <int kCtrl, int kRows, typename T>
+__device__ __forceinline__ T dpp_or_0(T v) {
+    if constexpr (sizeof(T) == 8) {
+        const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xF, true);
+        const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), kCtrl, kRows, 0xF, true);
+        return (T)(((uint64_t)hi << 32) | lo);
+    } else {
+        return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xF, true);
+    }
+}
+
+// Folds each lane's value with those of all lanes before it (0: neutral): row
+// shifts by 1, 2, 4 and 8, then the rows' last lanes broadcast to the rows
+// after them.  (With LDS shuffles instead, two per step for a 64-bit sum, a
+// ragged decode of 13 us took 0.3 us longer.)
+template <typename T, typename F>
+__device__ __forceinline__ T wave_fold(T v, F&& f) {
+    v = f(v, dpp_or_0<0x111, 0xF>(v));
+    v = f(v, dpp_or_0<0x112, 0xF>(v));
+    v = f(v, dpp_or_0<0x114, 0xF>(v));
+    v = f(v, dpp_or_0<0x118, 0xF>(v));
+    v = f(v, dpp_or_0<0x142, 0xA>(v));
+    return f(v, dpp_or_0<0x143, 0xC>(v));
+}
+
 // Exclusive prefix sum of one value per thread over a workgroup of kThreads.
-template <int kThreads, typename T>
+// kAgain: another scan in s_wave follows (else a barrier does before s_wave's
+// memory is written again).
+template <int kThreads, bool kAgain, typename T>
 __device__ __forceinline__ T block_exclusive_scan(T v, T* s_wave, T* total) {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    T incl = v;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const T t = __shfl_up(incl, d, kWave);
-        if (lane >= d) incl += t;
-    }
+    const T incl = wave_fold(v, [](T a, T b) { return a + b; });
     if (lane == kWave - 1) s_wave[wave] = incl;
     __syncthreads();
     T base = 0, all = 0;
@@ -483,7 +507,7 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* s_wave, T* total) {
         base += (w < wave) ? s_wave[w] : 0;
         all += s_wave[w];
     }
-    __syncthreads();   // s_wave is reused by the next scan
+    if constexpr (kAgain) __syncthreads();
     *total = all;
     return base + incl - v;
 }
@@ -502,8 +526,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(DecodeParams 
         if (sort) s_rem[b] = len % p.chunk;
     }
     int n_full, n_part;
-    int pos_f = block_exclusive_scan<kPlanThreads>(nf, s_wave, &n_full);
-    int pos_p = block_exclusive_scan<kPlanThreads>(np, s_wave, &n_part);   // also publishes s_rem (barriers inside)
+    int pos_f = block_exclusive_scan<kPlanThreads, true>(nf, s_wave, &n_full);
+    int pos_p = block_exclusive_scan<kPlanThreads, true>(np, s_wave, &n_part);   // also publishes s_rem (barriers inside)
     if (tid == 0) work[0] = n_full + n_part;
     for (int b = tid; b < p.batch; b += kPlanThreads) {
         const int len = clamp_len(p, b);
@@ -555,6 +579,10 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(DecodeParams 
 // Hkv = 8, bf16 pages: 88.5 -> 30.3 us; 64 of up to 32768, Hq = 64, fp8 pages:
 // 395.8 -> 360.9 us.
 //
+// Cutting sequences costs a second item per team and the combine.  Where whole
+// sequences are nearly as even (kWholeSlack), a team takes `per` of them in a
+// row, and nothing is left to combine.
+//
 // A split length given by the caller keeps the work list (p.work): a fixed
 // grid walks its entries, each once per kv head or pair (the head fastest, so
 // heads of one split run together).
@@ -574,6 +602,17 @@ __device__ __forceinline__ int team_count(const DecodeParams& p, int64_t total) 
     return total < p.teams ? (int)total : p.teams;
 }
 
+// Blocks per team that the cuts cost: a team runs per = ceil(batch / teams)
+// whole sequences if per times the longest one is at most this much above an
+// even share, unless the batch has a block per team or less.  Equal lengths,
+// us cut / whole: 60 of 4096 (Hq = 128, Hkv = 8) 170.6 / 155.7; Hq = 32,
+// Hkv = 8, 16-token pages: 60 of 1024 48.9 / 43.0, 20 of 512 (2.75 above)
+// 21.6 / 17.8, but 20 of 1024 (5.5 above) 26.7 / 30.0; 2 of 512 with Hq = 16,
+// Hkv = 2 (8 blocks, 256 teams) 13.9 / 15.5.
+constexpr int kWholeSlack = 4;
+// The prefix's total then.
+constexpr int64_t kWholeTeams = -1;
+
 __device__ __forceinline__ int seq_blocks(int len) {
     return (len + plan::kDecodeStepRound - 1) / plan::kDecodeStepRound;
 }
@@ -590,43 +629,65 @@ __global__ __launch_bounds__(kPair ? 2 * kDecThreads : kDecThreads) void decode_
     // work list: items blockIdx.x, + gridDim.x, ...
     int item = blockIdx.x;
     const int n_items = p.work != nullptr ? p.work[0] * per_entry : 0;
-    // teams: blocks [g0, g1) of the batch, the first of them block `blk` of sequence b
+    // teams: blocks [g0, g1) of the batch, the first of them block `blk` of
+    // sequence b, and none of sequence b_end
     const int team = blockIdx.x / per_entry;
     int64_t g0 = 0, g1 = 0;
-    int b = 0, blk = 0;
+    int b = 0, b_end = p.batch, blk = 0;
     if (p.work == nullptr) {
         int64_t* s_wave = reinterpret_cast<int64_t*>(smem);
         int* s_pos = reinterpret_cast<int*>(s_wave + kThreads / kWave);
+        int* s_max = s_pos + 2;   // per wave
         const int per = (p.batch + kThreads - 1) / kThreads;
         const int b_lo = min((int)threadIdx.x * per, p.batch), b_hi = min(b_lo + per, p.batch);
         int64_t sum = 0, total;
-        for (int i = b_lo; i < b_hi; ++i) sum += seq_blocks(clamp_len(p, i));
-        int64_t at = block_exclusive_scan<kThreads>(sum, s_wave, &total);
+        int longest = 0;
+        for (int i = b_lo; i < b_hi; ++i) {
+            const int n = seq_blocks(clamp_len(p, i));
+            sum += n;
+            longest = max(longest, n);
+        }
+        longest = wave_fold(longest, [](int x, int y) { return max(x, y); });   // (all of it in the last lane)
+        if ((threadIdx.x & (kWave - 1)) == kWave - 1) s_max[threadIdx.x / kWave] = longest;   // published by the scan's barrier
+        int64_t at = block_exclusive_scan<kThreads, false>(sum, s_wave, &total);
         // (uniform: the compiler does not see it through the LDS sum)
         total = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(total >> 32)) << 32) |
                           (uint32_t)__builtin_amdgcn_readfirstlane((int)total));
+        longest = 0;
+#pragma unroll
+        for (int w = 0; w < kThreads / kWave; ++w) longest = max(longest, s_max[w]);
+        longest = __builtin_amdgcn_readfirstlane(longest);
+        const int whole_per = (p.batch + p.teams - 1) / p.teams;
+        const bool whole_seqs = total > p.teams && (int64_t)whole_per * longest * p.teams <=
+                                                        total + (int64_t)kWholeSlack * p.teams;
+        if (blockIdx.x == 0 && threadIdx.x == 0) p.prefix[p.batch] = whole_seqs ? kWholeTeams : total;
         const int teams = team_count(p, total);
-        if (team < teams) {
+        if (whole_seqs) {
+            b = min(team * whole_per, p.batch);
+            b_end = min(b + whole_per, p.batch);
+            g1 = total;   // (b_end ends the range)
+        } else if (team < teams) {
             g0 = team_start(total, teams, team);
             g1 = team_start(total, teams, team + 1);
         }
-        const bool here = g0 >= at && g0 < at + sum;   // exactly one thread's, unless g0 is the end
-        if (here || blockIdx.x == 0) {
-            for (int i = b_lo; i < b_hi; ++i) {
-                const int n = seq_blocks(clamp_len(p, i));
-                if (blockIdx.x == 0) p.prefix[i] = at;
-                if (g0 >= at && g0 < at + n) {
-                    s_pos[0] = i;
-                    s_pos[1] = (int)(g0 - at);
+        if (!whole_seqs) {
+            const bool here = g0 >= at && g0 < at + sum;   // exactly one thread's, unless g0 is the end
+            if (here || blockIdx.x == 0) {
+                for (int i = b_lo; i < b_hi; ++i) {
+                    const int n = seq_blocks(clamp_len(p, i));
+                    if (blockIdx.x == 0) p.prefix[i] = at;
+                    if (g0 >= at && g0 < at + n) {
+                        s_pos[0] = i;
+                        s_pos[1] = (int)(g0 - at);
+                    }
+                    at += n;
                 }
-                at += n;
             }
+            if (g0 >= g1) return;
+            __syncthreads();
+            b = __builtin_amdgcn_readfirstlane(s_pos[0]);
+            blk = __builtin_amdgcn_readfirstlane(s_pos[1]);
         }
-        if (blockIdx.x == 0 && threadIdx.x == 0) p.prefix[p.batch] = total;
-        if (g0 >= g1) return;
-        __syncthreads();
-        b = __builtin_amdgcn_readfirstlane(s_pos[0]);
-        blk = __builtin_amdgcn_readfirstlane(s_pos[1]);
     }
     while (true) {
         int kvh, t_begin, t_end;
@@ -645,7 +706,7 @@ __global__ __launch_bounds__(kPair ? 2 * kDecThreads : kDecThreads) void decode_
             slot = ((int64_t)b * p.hkv + kvh) * p.nsplit + split;
             item += gridDim.x;
         } else {
-            if (g0 >= g1) break;
+            if (g0 >= g1 || b >= b_end) break;
             const int len = clamp_len(p, b);
             const int nb = seq_blocks(len);
             if (nb == 0) {   // empty sequences: the combine writes their O
@@ -715,7 +776,10 @@ __global__ __launch_bounds__(kDecThreads) void decode_combine_kernel(DecodeParam
         n = 0;
         first = base = step = 0;
         if (len > 0) {
+            // (both loads before the test: one memory round trip)
             const int64_t total = p.prefix[p.batch], g0 = p.prefix[b], g1 = g0 + seq_blocks(len);
+            asm volatile("" :: "s"(g0));
+            if (total == kWholeTeams) return;   // the whole workgroup: pass 1 wrote every output
             const int teams = team_count(p, total);
             auto team_of = [&](int64_t g) {   // the last team whose start is at most g
                 int t = (int)(g * teams / total);
