@@ -27,6 +27,7 @@
 // step was the bound: 150 us without any gather) at two waves per SIMD, and
 // every list was sorted (37 us): 224 us.  Three waves per SIMD: 165 VGPRs, 11.3
 // KB of LDS.
+#include <limits.h>
 #include <math.h>
 #include <stdint.h>
 
@@ -53,6 +54,7 @@ struct SparseParams {
     int n_hg;                   // ceil(group / 16) head groups per position
     int64_t n_items;            // batch * hkv * sq * n_hg
     int n_windows, window_shift;   // key windows a list is ordered by, 2^window_shift keys each
+    int sorted;                    // kSpFar: ordered by key instead
     FastDiv div_hg, div_sq, div_hkv;
     float scale_log2;           // |scale| * log2(e)
     uint32_t q_sign;            // 0x80008000 when scale < 0 (Q is negated on load)
@@ -60,7 +62,7 @@ struct SparseParams {
 
 constexpr int kSpWaves = 4;                  // waves (= work items) per workgroup
 constexpr int kSpStep = 32;                  // index entries per step
-constexpr int kSpRow = 288;                  // K / V row stride in LDS (256 + 32 bytes)
+constexpr int kSpRow = 288;                  // V row stride in LDS (256 + 32 bytes)
 constexpr int kSpTileBytes = kSpStep * kSpRow;
 constexpr int kSpList = 512;                 // index entries taken (and ordered) at a time
 constexpr int kSpWaveBytes = kSpTileBytes + kSpList * 4 + 16;   // 11.3 KB of LDS per wave (and a word to drop entries in)
@@ -76,15 +78,28 @@ constexpr float kSpMaxP = 65536.f;           // a lane's P of one step, before t
 // Up to 8192 keys all K/V fit: one window.
 constexpr int kSpWindowLog2 = 11;
 constexpr int kSpNoWindows = 8192;
-// Two waves per SIMD instead of three (kPerSimd below): a wave's next K rows are
-// gathered before its scores instead of after them (188 registers).  Chosen
-//  - for grids that fit the chip at two workgroups per CU, where a launch is one
-//    wave's chain of steps: S = 546, 512 entries 19.2 against 21.3 us, S = 2048,
-//    512 entries 29.2 against 31.1; at S = 3000 (750 workgroups) 15.3 against 14.6;
-//  - past 32768 keys, where L2 serves fewer waves better: 65536 keys, 512 entries
-//    1202 against 1371 us (the former kernel, sorted lists and two steps in
-//    flight: 1182), 1024 entries 2582 against 2729; 16384 keys: 199 against 188.
-constexpr int kSpManyKeys = 32768;
+// The kernel's forms.
+//  - kSpThree: three waves per SIMD (165 registers), a step of rows in flight.
+//  - kSpChain: two waves; a wave's next K rows are gathered before its scores
+//    instead of after them (188 registers).  For grids that fit the chip at two
+//    workgroups per CU, where a launch is one wave's chain of steps: S = 546,
+//    512 entries 19.2 against 21.3 us, S = 2048, 512 entries 29.2 against 31.1;
+//    at S = 3000 (750 workgroups) 15.3 against 14.6.
+//  - kSpFar: two waves, two steps of rows in flight (249 registers).  For rows
+//    that see more than 16384 keys on average (half of them under the causal
+//    mask), where L2 serves fewer waves better, and lists of 256 entries or
+//    more.  us, three waves / far: 24576 keys, full, 256 entries 291 / 272, 1024
+//    entries 813 / 675; 32768 keys, full, 512 entries 634 / 556; 40000 keys,
+//    causal, 512 entries 624 / 613; but 24576 keys, causal, 512 entries 316 /
+//    337, and 40000 keys, full, 64 entries 196 / 203.
+enum SpForm { kSpThree, kSpChain, kSpFar };
+constexpr int kSpFarKeys = 16384;
+constexpr int kSpFarList = 256;
+// kSpFar takes lists of 257 to 512 entries in full key order instead of by
+// windows: 65536 keys, 512 entries 1628 against 1635 us (full) and 1179 against
+// 1208 (causal), 40000 keys, full 771 against 801; but 256 entries at 24576 keys
+// 288 against 274, and 1024 entries (two parts) at 65536 keys 3354 against 3298.
+constexpr int kSpSortMin = 257;
 
 // Gathers read whole rows per instruction, in pieces of a quad (K, 64 bytes) or
 // of 16 lanes (V, 256 bytes); both run at the same rate (129-132 us for 4.3 GB
@@ -146,11 +161,57 @@ __device__ __forceinline__ void sp_transpose_quad(uint32_t& a0, uint32_t& a1, ui
         : "vcc", "scc");
 }
 
+// The value of lane ^ d: DPP quad permutes for d = 1, 2, a bit-mode swizzle
+// inside each half-wave for 4 <= d <= 16, the half-wave swap for 32.
+__device__ __forceinline__ int sp_xor(int v, int d, int lane) {
+    switch (d) {
+        case 1: return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+        case 2: return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+        case 4: return __builtin_amdgcn_ds_swizzle(v, (4 << 10) | 0x1F);
+        case 8: return __builtin_amdgcn_ds_swizzle(v, (8 << 10) | 0x1F);
+        case 16: return __builtin_amdgcn_ds_swizzle(v, (16 << 10) | 0x1F);
+        default: {
+            const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+            return (int)(lane < 32 ? r[1] : r[0]);
+        }
+    }
+}
+
+// Ascending bitonic sort of a wave's 512 ints, value 8*lane + r in x[r]:
+// distances of 8 values or more pair registers across lanes, smaller ones
+// pair registers of a lane.  Deterministic (no atomics).
+__device__ __forceinline__ void sp_sort512(int (&x)[8], int lane) {
+#pragma unroll
+    for (int k = 2; k <= 512; k <<= 1)
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            if (j >= 8) {
+                // value e pairs with e ^ j: same register of lane ^ (j / 8);
+                // the block of size k holding e sorts up when (e & k) == 0
+                const int d = j >> 3;
+                const bool keep_min = ((lane & d) == 0) == ((lane & (k >> 3)) == 0);
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    const int o = sp_xor(x[r], d, lane);
+                    x[r] = keep_min ? min(x[r], o) : max(x[r], o);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    if (r & j) continue;
+                    const bool up = ((8 * lane + r) & k) == 0;
+                    const int lo = min(x[r], x[r | j]), hi = max(x[r], x[r | j]);
+                    x[r] = up ? lo : hi;
+                    x[r | j] = up ? hi : lo;
+                }
+            }
+        }
+}
+
 // kSameRows: K and V rows are the same number of bytes apart, so one offset
-// (kept in the list instead of the key) addresses both.  kPerSimd: waves per
-// SIMD, see kSpManyKeys.
-template <bool kSameRows, int kPerSimd>
-__global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_kernel(SparseParams p) {
+// (kept in the list instead of the key) addresses both.
+template <bool kSameRows, SpForm kForm>
+__global__ __launch_bounds__(kSpWaves * kWave, kForm == kSpThree ? 3 : 2) void sparse_prefill_kernel(SparseParams p) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[kSpWaves * kSpWaveBytes];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -223,8 +284,10 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
     // 16tt + l16 in lane l16, the MFMA's A operand with dims 32g + 8ks .. +7 in
     // register ks.  V: instruction i, group g reads entry 8g + i, a row per 16
     // lanes, into the same row of the LDS tile.
-    u32x4_t kr[2][4], vr[8];
-    auto issue_k = [&](int t) {
+    struct Rows {
+        u32x4_t k[2][4], v[8];
+    };
+    auto issue_k = [&](int t, u32x4_t (&kr)[2][4]) {
         const u32x4_t* w = reinterpret_cast<const u32x4_t*>(il + t * kSpStep + (l16 & 12));
         const u32x4_t r0 = w[0], r1 = w[4];
         const uint32_t chunk = (uint32_t)(g * 64 + (lane & 3) * 16);
@@ -234,7 +297,7 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
             kr[1][i] = buf_load16(krs, (kSameRows ? r1[i] : r1[i] * kss) + chunk);
         }
     };
-    auto issue_v = [&](int t) {
+    auto issue_v = [&](int t, u32x4_t (&vr)[8]) {
         const u32x4_t* w = reinterpret_cast<const u32x4_t*>(il + t * kSpStep + g * 8);
         const u32x4_t r0 = w[0], r1 = w[1];
 #pragma unroll
@@ -251,7 +314,7 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i][d] = a[i], o[i][d + 1] = b[i];
     };
-    auto stage_v = [&]() {
+    auto stage_v = [&](const u32x4_t (&vr)[8]) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(tile + (8 * g + i) * kSpRow + l16 * 16) = vr[i];
     };
@@ -285,8 +348,8 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
     };
     for (int c0 = 0; c0 < p.nsparse; c0 += kSpList) {
         // Up to 512 entries, the usable ones first and window by window
-        // (a fixed order, by slot modulo 8 and then lane, in a window).  The
-        // order of the sum changes by rounding only.
+        // (a fixed order, by slot modulo 8 and then lane, in a window) or
+        // sorted.  The order of the sum changes by rounding only.
         int x[8];
         {
             const u32x4_t a0 = buf_load16(irs, (uint32_t)(c0 + 8 * lane) * 4);
@@ -302,7 +365,18 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
         int at[8], n_valid = 0;
 #pragma unroll
         for (int r = 0; r < 8; ++r) at[r] = kSpList;   // unusable: dropped
-        for (int w = 0; w < p.n_windows; ++w) {
+        const bool sorted = kForm == kSpFar && p.sorted;
+        if (sorted) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) x[r] = x[r] < 0 ? INT_MAX : x[r];
+            sp_sort512(x, lane);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                n_valid += __builtin_popcountll(__builtin_amdgcn_ballot_w64(x[r] != INT_MAX));
+                at[r] = x[r] != INT_MAX ? 8 * lane + r : kSpList;
+            }
+        }
+        for (int w = 0; w < (sorted ? 0 : p.n_windows); ++w) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
                 const bool in = (x[r] >> p.window_shift) == w;
@@ -321,18 +395,17 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
 #pragma unroll
         for (int r = 0; r < 8; ++r) il[at[r]] = kSameRows ? (int)((uint32_t)x[r] * kss) : x[r];
         const int steps = (n_valid + kSpStep - 1) / kSpStep;
-        issue_k(0);
-        issue_v(0);
-        for (int t = 0; t < steps; ++t) {
-            const bool more = t + 1 < steps;
+        constexpr int kAhead = kForm == kSpFar ? 2 : 1;   // steps of rows in flight
+        auto step = [&](int t, Rows& rows) {
+            const bool more = t + kAhead < steps;
             u32x4_t kt[2][4];
-            u32x4_t(&ka)[2][4] = kPerSimd == 2 ? kt : kr;   // (three waves: in place, no registers to spare)
+            u32x4_t(&ka)[2][4] = kForm == kSpChain ? kt : rows.k;   // (else in place, no registers to spare)
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-                for (int d = 0; d < 4; d += 2) transpose(kr[tt], ka[tt], d);
-            if constexpr (kPerSimd == 2) {
-                if (more) issue_k(t + 1);
+                for (int d = 0; d < 4; d += 2) transpose(rows.k[tt], ka[tt], d);
+            if constexpr (kForm == kSpChain) {
+                if (more) issue_k(t + kAhead, rows.k);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
@@ -341,12 +414,12 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) s[tt] = mfma16(as_bf16x8(ka[tt][ks]), qop[ks], s[tt]);
             }
-            if constexpr (kPerSimd == 3) {
-                if (more) issue_k(t + 1);
+            if constexpr (kForm != kSpChain) {
+                if (more) issue_k(t + kAhead, rows.k);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            stage_v();
-            if (more) issue_v(t + 1);
+            stage_v(rows.v);
+            if (more) issue_v(t + kAhead, rows.v);
             const int nv = n_valid - t * kSpStep;
             if (nv < kSpStep) {
 #pragma unroll
@@ -382,6 +455,22 @@ __global__ __launch_bounds__(kSpWaves * kWave, kPerSimd) void sparse_prefill_ker
                 const bf16x4_t hi = lds_read_tr16(reinterpret_cast<const __bf16*>(vrd + 16 * kSpRow + dt * 32));
                 oacc[dt] = mfma16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pop, oacc[dt]);
             }
+        };
+        Rows ra;
+        issue_k(0, ra.k);
+        issue_v(0, ra.v);
+        if constexpr (kForm == kSpFar) {
+            Rows rb;
+            if (steps > 1) {
+                issue_k(1, rb.k);
+                issue_v(1, rb.v);
+            }
+            for (int t = 0; t < steps; t += 2) {
+                step(t, ra);
+                if (t + 1 < steps) step(t + 1, rb);
+            }
+        } else {
+            for (int t = 0; t < steps; ++t) step(t, ra);
         }
     }
 
@@ -465,12 +554,14 @@ extern "C" int fgqa_sparse_prefill_bf16(const fgqa_sparse_prefill_args* a, void*
     const dim3 grid((unsigned)blocks), threads(kSpWaves * kWave);
     const int cus = device_cu_count();
     if (cus <= 0) return FGQA_ERR_HIP;
-    const bool few = p.skv > kSpManyKeys || blocks <= 2 * cus;
-    const bool same = p.k_ss == p.v_ss;
-    if (few && same) hipLaunchKernelGGL((sparse_prefill_kernel<true, 2>), grid, threads, 0, s, p);
-    else if (few) hipLaunchKernelGGL((sparse_prefill_kernel<false, 2>), grid, threads, 0, s, p);
-    else if (same) hipLaunchKernelGGL((sparse_prefill_kernel<true, 3>), grid, threads, 0, s, p);
-    else hipLaunchKernelGGL((sparse_prefill_kernel<false, 3>), grid, threads, 0, s, p);
+    const bool few = blocks <= 2 * cus;
+    const bool far = !few && p.nsparse >= kSpFarList && (p.causal ? p.skv / 2 : p.skv) > kSpFarKeys;
+    p.sorted = p.nsparse >= kSpSortMin && p.nsparse <= kSpList;
+    using Kernel = void (*)(SparseParams);
+    const Kernel fns[3][2] = {{sparse_prefill_kernel<false, kSpThree>, sparse_prefill_kernel<true, kSpThree>},
+                              {sparse_prefill_kernel<false, kSpChain>, sparse_prefill_kernel<true, kSpChain>},
+                              {sparse_prefill_kernel<false, kSpFar>, sparse_prefill_kernel<true, kSpFar>}};
+    hipLaunchKernelGGL(fns[few ? kSpChain : far ? kSpFar : kSpThree][p.k_ss == p.v_ss], grid, threads, 0, s, p);
     if (hipGetLastError() != hipSuccess) return FGQA_ERR_HIP;
     return FGQA_OK;
 }
