@@ -89,6 +89,11 @@ enum fgqa_kernel_choice {
  *            yields O = 0 and lse = -inf.
  *   scale  multiplies q.k (the reference passes 1/sqrt(D)).
  *   split_tokens  KV tokens per split (rounded up to 128); 0 = automatic.
+ *            A ragged call (seqlens) with 0 cuts the sequences where the whole
+ *            batch's tokens are shared out evenly, so a sequence's result may
+ *            differ by rounding with the lengths of the others in the batch (it
+ *            is the same from call to call).  A given split_tokens cuts each
+ *            sequence by itself: the same bits in any batch.
  *   workspace / workspace_bytes  device scratch of at least
  *            fgqa_decode_workspace_bytes(); pass NULL/0 to let the library use
  *            its own per-device cached buffer (allocated on first use).  Calls
