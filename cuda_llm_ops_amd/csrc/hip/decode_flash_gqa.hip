@@ -733,7 +733,8 @@ __global__ __launch_bounds__(kPair ? 2 * kDecThreads : kDecThreads) void decode_
 
 // Launches pass 1 over a ragged batch: the head-pair form (one 8-wave
 // workgroup per CU) when the kv heads pair up, else two 4-wave workgroups per
-// CU.  Persistent: the grid never exceeds what the CUs hold at once.
+// CU.  A work list's grid never exceeds what the CUs hold at once; the teams fill
+// 256 CUs (kDecodeItemSlots), and on fewer they run in more than one round.
 template <int kKv, int kSeg>
 static void launch_list(const DecodeParams& p, int nsplit, int cus, hipStream_t s) {
     const bool pair = (p.hkv % 2) == 0;
@@ -753,7 +754,7 @@ static void launch_list(const DecodeParams& p, int nsplit, int cus, hipStream_t 
 // slots past the last re-read it and are masked), then one merge of the ways
 // through LDS.  A workgroup holds 16 / kWays heads.  The launch is bound by
 // memory round trips, one per batch, so the host picks as many ways as one
-// batch each needs (combine_ways).  With one way per head at 128 partials (one
+// batch each needs (launch_combine).  With one way per head at 128 partials (one
 // 32768-token sequence, Hq = 64, Hkv = 8): 27.4 us; 16 ways: 4.3 us.
 template <bool kTeam, int kWays>
 __global__ __launch_bounds__(kDecThreads) void decode_combine_kernel(DecodeParams p) {

@@ -354,7 +354,7 @@ int validate_prefill(const fgqa_prefill_args* a) {
     }
     if (a->batch == 0 || a->seqlen_q == 0) return FGQA_OK;
     if (a->q == nullptr || a->k == nullptr || a->v == nullptr || a->o == nullptr) return FGQA_ERR_INVALID_ARGUMENT;
-    // the copies are made with 2-byte accesses: any alignment and strides
+    // the copies need no alignment: any addresses and strides
     if (padded) return FGQA_OK;
     if (!aligned16(a->q) || !aligned16(a->k) || !aligned16(a->v) || !aligned16(a->o)) return FGQA_ERR_UNSUPPORTED;
     // (O rows go out as 16-byte stores, so O's strides need 8 elements too)
@@ -439,8 +439,8 @@ static int choice_native64(const fgqa_prefill_args* a, int64_t units, int64_t cu
 //    its units mostly padding.  Then the split kernel only for long sequences
 //    (S = 6000, 752 units 272 / 259 / 270; S = 520, 544 units 33 / 43 / 37).
 //    Grids of more than 32 units per CU keep the whole-range kernel, which
-//    fgqa_prefill_kernel_choice has always reported for them (64 per CU: 16.0
-//    ms against 14.1).
+//    fgqa_prefill_kernel_choice has always reported for them (32 is no measured
+//    line: at 64 per CU whole takes 16.0 ms and wide 14.1).
 static int choice_short_or_full(const fgqa_prefill_args* a, int64_t units, int64_t cus) {
     const int64_t s = longest_row(a), tiles = ceil_div(s, 64), wu = wide_units(a);
     if (units <= cus) return tiles <= 5 || tiles == 7 ? FGQA_KERNEL_WHOLE : FGQA_KERNEL_AUTO;
@@ -634,7 +634,7 @@ int validate_backward_pointers(const fgqa_prefill_backward_args* a) {
         return FGQA_ERR_INVALID_ARGUMENT;
     if (a->seqlen_kv > 0 && (a->k == nullptr || a->v == nullptr || a->grad_k == nullptr || a->grad_v == nullptr))
         return FGQA_ERR_INVALID_ARGUMENT;
-    // padded head dims: the copies are made with 2-byte accesses
+    // padded head dims: the copies need no alignment
     if (backward_padded(a)) return FGQA_OK;
     const void* ptrs[8] = {a->q, a->k, a->v, a->o, a->grad_o, a->grad_q, a->grad_k, a->grad_v};
     for (const void* ptr : ptrs)

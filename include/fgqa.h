@@ -249,7 +249,9 @@ int fgqa_decode_paged(const fgqa_decode_paged_args* args, void* stream);
  *           alignment nor strides in multiples of 8.  (Pairs with both dims
  *           up to 64 and multiples of 8, with aligned tensors and strides in
  *           multiples of 8, run kernels built for 64 in place, except
- *           FGQA_KERNEL_TALL.)  Head dims above 256
+ *           FGQA_KERNEL_TALL and calls whose O lies over an input; those that
+ *           merge nothing touch no workspace, though the size query counts the
+ *           copies.)  Head dims above 256
  *           return FGQA_ERR_UNSUPPORTED, and so do a window or sink with
  *           head_dim 192 and FGQA_KERNEL_SPLIT / _WIDE / _TALL with q/k
  *           padded to 256.
@@ -356,8 +358,8 @@ int fgqa_prefill_kernel_name(const fgqa_prefill_args* args, const char** name);
  *   grad_k have 192-element rows, v, o, grad_o, grad_v 128-element rows.
  *   Built: (128, 128), and (192, 128) without a window.  Q/K head dims up to
  *   128 (or 192, without a window) with V/O head dims up to 128 run on copies
- *   of q, k, v, o, grad_o zero-padded to a built pair (element by element:
- *   no alignment needed), the first columns of the padded gradients copied
+ *   of q, k, v, o, grad_o zero-padded to a built pair (no alignment needed;
+ *   aligned rows are copied 16 bytes at a time), the first columns of the padded gradients copied
  *   out; the copies live in the workspace after the built call's own bytes
  *   (fgqa_prefill_backward_workspace_bytes includes them).  Other head dims
  *   return FGQA_ERR_UNSUPPORTED.
