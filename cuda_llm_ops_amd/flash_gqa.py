@@ -430,12 +430,14 @@ def _uses_no_scratch(a) -> bool:
     """The call runs at a head dim up to 64 on the tensors themselves and merges
     nothing, so the copies that the size query counts are not made: dims,
     addresses and strides in multiples of 8 elements, O apart from the inputs
-    (else the library makes the copies), and no causal grid of at most 256 units
-    of 256 rows (others never merge)."""
+    (else the library makes the copies), no causal grid of at most 256 units of
+    256 rows (others never merge), and neither rows nor keys missing (their
+    addresses may be null)."""
     dqk, dv = a.head_dim, a.head_dim_v or a.head_dim
     if dqk > 64 or dv > 64 or (dqk | dv) & 7 or a.kernel == _lib.FGQA_KERNEL_TALL:
         return False
-    if a.causal and a.batch * a.num_q_heads * a.seqlen_q <= 65536:
+    rows = a.batch * a.num_q_heads * a.seqlen_q
+    if rows == 0 or a.seqlen_kv == 0 or (a.causal and rows <= 65536):
         return False
     if (a.q | a.k | a.v | a.o) & 15 or any(s & 7 for st in (a.q_stride, a.k_stride, a.v_stride, a.o_stride) for s in st):
         return False

@@ -46,3 +46,16 @@ def test_no_scratch_in_place(cuda, D, causal):
     mine, device, _ = held(lambda: fg.flash_gqa_forward_bshd(q, k, v, out=room[..., :D], lse=lse, causal=causal))
     assert mine >= copies and device < 1 << 22
     impl._PREFILL_WORKSPACES.clear()
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_no_query_rows(cuda, causal):
+    """Nothing to do, with keys enough that the size query is over 32 MB."""
+    import torch
+    import cuda_llm_ops_amd as fg
+    print(f"causal={causal}", flush=True)
+    q = torch.empty((1, 0, 16, 64), device=cuda, dtype=torch.bfloat16)
+    k = torch.zeros((1, 8192, 16, 64), device=cuda, dtype=torch.bfloat16)
+    out, lse = fg.flash_gqa_forward_bshd(q, k, k, causal=causal)
+    torch.cuda.synchronize()
+    assert out.shape == (1, 0, 16, 64) and lse.shape == (1, 16, 0)
