@@ -20,13 +20,14 @@
 // The next step's K and V rows are in flight while a step is computed.
 //
 // What bounds it: each step gathers 16 KB of K/V rows and does little with
-// them.  At S = 16384, 512 entries (4.3 GB of gathers) the gathers alone take
+// them.  (Kernel times on one set of lists, repeated; calls on alternating inputs
+// take some 10 us more.)  At S = 16384, 512 entries (4.3 GB of gathers) the gathers alone take
 // 129 us when they all hit L1, the steps without gathers 112 us; together 155 us
 // from L1 and 189 us from the real lists (L2 misses; 4 MB of L2 per XCD against
 // 8 MB of K/V).  Before, K went through LDS as well (32 KB of LDS traffic per
 // step was the bound: 150 us without any gather) at two waves per SIMD, and
 // every list was sorted (37 us): 224 us.  Three waves per SIMD: 165 VGPRs, 11.3
-// KB of LDS.
+// KB of LDS.  Other forms for small grids and for many keys: SpForm below.
 #include <limits.h>
 #include <math.h>
 #include <stdint.h>
